@@ -11,10 +11,12 @@
  *   - split-K rows (narrow N, long K: fp32 partial sums of k ranges, reduced by a second kernel
  *     on the same stream) need a workspace of tempo_gemm_*_workspace_bytes() bytes.  The launch
  *     entry points take it from the library's pool: one device buffer per (device, stream),
- *     allocated with hipMalloc the first time a shape needs it and grown (after a synchronise of
- *     that stream) when a larger one does.  So the first split-K call on a stream allocates;
- *     later calls of the same or smaller shapes do not.  Calls on different streams never
- *     share a workspace.  Every other row uses no workspace and allocates nothing.
+ *     allocated with hipMalloc the first time a shape needs it and grown when a larger one does
+ *     (the outgrown buffer is kept: nothing is synchronised).  So the first split-K call on a
+ *     stream allocates; later calls of the same or smaller shapes do not.  Calls on different
+ *     streams never share a workspace, and threads may call on one stream at once: a call holds
+ *     the buffer's lock until its last kernel is enqueued.  Every other row uses no workspace and
+ *     allocates nothing.
  *   - the int returned is a hipError_t value: 0 = success; TEMPO_FALLBACK (9, the value of
  *     hipErrorInvalidConfiguration) = "shape not covered, take your own path" -- a legal
  *     answer, not a failure (reference kernels/shipped/gemm_fp16/sm_70/dispatch.inc:12-13,26).

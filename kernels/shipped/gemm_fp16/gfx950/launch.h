@@ -212,10 +212,12 @@ inline hipError_t launch_line_impl(const GemmParams& p, hipStream_t s, const Wor
     *w->need = bytes;
     return hipSuccess;
   }
+  Lease ws;
   if (a.ks > 1) {
     hipError_t werr = hipSuccess;
-    a.part = workspace_for(*w, bytes, s, &werr);
-    if (!a.part) return werr;
+    ws = workspace_for(*w, bytes, s, &werr);
+    if (!ws.ptr) return werr;
+    a.part = ws.ptr;
   }
   hipLaunchKernelGGL((k_stream_line<MB, R, D, 0, EPI, SN, TPB>), dim3(wgs * a.ks),
                      dim3(64 * SN * a.S), lds, s, a, G);

@@ -28,14 +28,14 @@ hipError_t launch_ilv(const GemmParams& p, hipStream_t s, const Workspace& w) {
   }
   if constexpr (SW > 0) {
     hipError_t werr = hipSuccess;
-    float* ws = workspace_for(w, bytes, s, &werr);
-    if (!ws) return werr;
+    const Lease ws = workspace_for(w, bytes, s, &werr);
+    if (!ws.ptr) return werr;
     hipLaunchKernelGGL((k_gemm_ilv<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, 1>),
                        dim3(nm * nn * splits), blk, 0, s, p.A, p.B, p.C, p.M, p.N, p.K, p.lda, p.ldb,
-                       p.ldc, ws, splits, p.N);
+                       p.ldc, ws.ptr, splits, p.N);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_reduce(ws, splits, p.M, p.N, p.C, p.ldc, s);
+    return launch_reduce(ws.ptr, splits, p.M, p.N, p.C, p.ldc, s);
   }
   return hipErrorInvalidConfiguration;  // not reached: splits == 1 where SW == 0
 }
@@ -132,13 +132,13 @@ hipError_t launch_ilv_planned(const GemmParams& p, hipStream_t s, const Workspac
     *w.need = bytes;
     return hipSuccess;
   }
-  float* ws = nullptr;
+  Lease ws;
   if (bytes) {
     hipError_t err = hipSuccess;
     ws = workspace_for(w, bytes, s, &err);
-    if (!ws) pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, false);  // unsplit
+    if (!ws.ptr) pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, false);  // unsplit
   }
-  return run_plan<GROUP, XCD, RSP>(p, s, ws, pl, gate_up);
+  return run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, gate_up);
 }
 
 template <int GROUP, int XCD, int RSP>
@@ -159,9 +159,12 @@ bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double
     *w.need = bytes;
     return true;
   }
-  float* ws = nullptr;
-  if (bytes && !(ws = workspace_for(w, bytes, s, e))) return false;
-  *e = run_plan<GROUP, XCD, RSP>(p, s, ws, pl, false);
+  Lease ws;
+  if (bytes) {
+    ws = workspace_for(w, bytes, s, e);
+    if (!ws.ptr) return false;
+  }
+  *e = run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, false);
   return true;
 }
 

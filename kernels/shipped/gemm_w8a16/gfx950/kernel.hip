@@ -2885,8 +2885,10 @@ __global__ __launch_bounds__(512, 1) void k_stream_phase(PhaseArgs p) {
 // A split-K row adds fp32 partial sums of its k ranges, [splits][M][N], in a workspace and reduces
 // them with k_splitk_reduce on the same stream.  The workspace is either memory the caller hands
 // over, or the delivery's pool: one buffer per (device, stream), allocated on first use and grown
-// when a larger shape needs it, so calls on different streams stay independent and calls on one
-// stream are ordered by it.
+// when a larger shape needs it, so calls on different streams stay independent.  A call is two
+// kernels, and a stream orders kernels, not calls: the pool's buffer is leased, locked from before
+// the first is enqueued until after the second, so that no other thread's partial sums land
+// between them.
 
 // Workspace of a split-K row.  `ptr`/`bytes`: device memory the caller hands over (may be
 // null / 0); `pool`: the row may take the delivery's per-(device, stream) pool instead; `need`:
@@ -2899,57 +2901,80 @@ struct Workspace {
   size_t* need = nullptr;
 };
 
+// The workspace of one call, from workspace_for() until the call's last kernel is enqueued.  ptr is
+// null where none could be had; `held` locks a pool buffer (nothing for the caller's memory).
+struct Lease {
+  float* ptr = nullptr;
+  std::unique_lock<std::mutex> held;
+};
+
 // The pool: one buffer per (device, stream), grown on demand.  A buffer that a larger shape
-// outgrows is retired, not freed: work already queued on the stream, a graph captured earlier
-// or another thread that took the pointer a moment ago may still use it, so it stays allocated
-// until the process ends.  Sizes are whole powers of two from 1 MiB, so the retired buffers of a
-// stream together stay below its current one.  Growing needs hipMalloc, which a stream under graph capture cannot take: there
-// the pool returns hipErrorStreamCaptureUnsupported and the caller hands over its workspace
-// instead (launch_with, or the C ABI's *_launch_ws entry points).  (The frozen file's preamble
-// includes <map>, <mutex>, <utility> and <vector>.)
-inline void* pool_buffer(hipStream_t s, size_t bytes, hipError_t* err) {
+// outgrows is retired, not freed: work already queued on the stream or a graph captured earlier
+// may still use it, so it stays allocated until the process ends.  Sizes are whole powers of two
+// from 1 MiB, so the retired buffers of a stream together stay below its current one.  Growing
+// needs hipMalloc, which a stream under graph capture cannot take: there the pool returns
+// hipErrorStreamCaptureUnsupported and the caller hands over its workspace instead (launch_with,
+// or the C ABI's *_launch_ws entry points).  (The frozen file's preamble includes <map>, <mutex>,
+// <utility> and <vector>.)
+struct PoolBuffer {
+  std::mutex busy;
+  void* ptr = nullptr;
+  size_t bytes = 0;
+  std::vector<void*> retired;
+};
+inline Lease pool_lease(hipStream_t s, size_t bytes, hipError_t* err) {
   static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, std::pair<void*, size_t>> pool;
-  static std::vector<void*> retired;
+  static std::map<std::pair<int, hipStream_t>, PoolBuffer> pool;  // nodes keep their address
+  Lease l;
   int dev = 0;
-  if ((*err = hipGetDevice(&dev)) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  std::pair<void*, size_t>& e = pool[std::make_pair(dev, s)];
-  if (e.second < bytes) {
+  if ((*err = hipGetDevice(&dev)) != hipSuccess) return l;
+  PoolBuffer* e = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    e = &pool[std::make_pair(dev, s)];
+  }
+  std::unique_lock<std::mutex> held(e->busy);
+  if (e->bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if ((*err = hipStreamIsCapturing(s, &cs)) != hipSuccess) return nullptr;
+    if ((*err = hipStreamIsCapturing(s, &cs)) != hipSuccess) return l;
     if (cs != hipStreamCaptureStatusNone) {
       *err = hipErrorStreamCaptureUnsupported;
-      return nullptr;
+      return l;
     }
     size_t size = (size_t)1 << 20;
     while (size < bytes) size *= 2;
     // another stream's capture, which would forbid this thread's hipMalloc, is none of its concern
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    if ((*err = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return nullptr;
+    if ((*err = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return l;
     void* q = nullptr;
     const hipError_t got = hipMalloc(&q, size);
     *err = hipThreadExchangeStreamCaptureMode(&mode);
     if (got != hipSuccess) {
       (void)hipGetLastError();  // the caller may go on without a workspace
       *err = hipErrorOutOfMemory;
-      return nullptr;
+      return l;
     }
-    if (e.first) retired.push_back(e.first);
-    e = std::make_pair(q, size);
+    if (e->ptr) e->retired.push_back(e->ptr);
+    e->ptr = q;
+    e->bytes = size;
   }
-  return e.first;
+  l.ptr = static_cast<float*>(e->ptr);
+  l.held = std::move(held);
+  return l;
 }
 
 // The workspace of a split-K launch: the caller's if it is large enough, else the pool's when the
-// row may take it.  nullptr with *err set otherwise (hipErrorOutOfMemory: the caller's buffer is
+// row may take it.  Null with *err set otherwise (hipErrorOutOfMemory: the caller's buffer is
 // too small and no pool was allowed).
-inline float* workspace_for(const Workspace& w, size_t bytes, hipStream_t s, hipError_t* err) {
+inline Lease workspace_for(const Workspace& w, size_t bytes, hipStream_t s, hipError_t* err) {
   *err = hipSuccess;
-  if (w.ptr && w.bytes >= bytes) return static_cast<float*>(w.ptr);
-  if (w.pool) return static_cast<float*>(pool_buffer(s, bytes, err));
-  *err = hipErrorOutOfMemory;
-  return nullptr;
+  if (w.pool && !(w.ptr && w.bytes >= bytes)) return pool_lease(s, bytes, err);
+  Lease l;
+  if (w.ptr && w.bytes >= bytes)
+    l.ptr = static_cast<float*>(w.ptr);
+  else
+    *err = hipErrorOutOfMemory;
+  return l;
 }
 
 // Split count of a split-K row: the most splits such that tiles x splits stays within `slots`

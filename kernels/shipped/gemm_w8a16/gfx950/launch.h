@@ -254,10 +254,12 @@ inline hipError_t launch_line_fmt(const W8A16Params& p, hipStream_t s, const Wor
     *w->need = bytes;
     return hipSuccess;
   }
+  Lease ws;
   if (a.ks > 1) {
     hipError_t werr = hipSuccess;
-    a.part = workspace_for(*w, bytes, s, &werr);
-    if (!a.part) return werr;
+    ws = workspace_for(*w, bytes, s, &werr);
+    if (!ws.ptr) return werr;
+    a.part = ws.ptr;
   }
   hipLaunchKernelGGL((k_stream_line<MB, R, D, BFMT, EPI, SN, TPB, TL>), dim3(wgs * a.ks),
                      dim3(64 * SN * a.S), lds, s, a, G);
@@ -397,8 +399,9 @@ inline hipError_t launch_phase_ks(const W8A16Params& p, hipStream_t s, const Wor
     return hipSuccess;
   }
   hipError_t werr = hipSuccess;
-  a.part = workspace_for(w, bytes, s, &werr);
-  if (!a.part) return werr;
+  const Lease ws = workspace_for(w, bytes, s, &werr);
+  if (!ws.ptr) return werr;
+  a.part = ws.ptr;
   constexpr int CUS = StreamPhase<MB, NS, D, 1, 0, 1>::CUS, NWV = StreamPhase<MB, NS, D, 1, 0, 1>::NWV;
   if (p.fmt == 1)
     hipLaunchKernelGGL((k_stream_phase<MB, NS, D, 1, 0, 1>), dim3(CUS), dim3(64 * NWV), lds, s, a);
@@ -594,10 +597,11 @@ inline bool phase_instead(const W8A16Params& p, hipStream_t s, const Workspace& 
     *w.need = std::max(bytes, own_bytes);
     return true;
   }
+  const Lease lease = workspace_for(w, bytes, s, e);
+  if (!lease.ptr) return false;
   Workspace ws;
-  ws.ptr = workspace_for(w, bytes, s, e);
+  ws.ptr = lease.ptr;
   ws.bytes = bytes;
-  if (!ws.ptr) return false;
   *e = ks == 4   ? launch_phase_slabs<MB, 4>(p, s, ws)
        : ks == 2 ? launch_phase_slabs<MB, 2>(p, s, ws)
                  : launch_phase_slabs<MB, 8>(p, s, ws);

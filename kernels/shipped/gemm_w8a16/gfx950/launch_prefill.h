@@ -36,16 +36,16 @@ hipError_t launch_ilv8(const W8A16Params& p, hipStream_t s, const Workspace& w) 
   }
   if constexpr (SW > 0) {
     hipError_t werr = hipSuccess;
-    float* ws = workspace_for(w, bytes, s, &werr);
-    if (!ws) return werr;
+    const Lease ws = workspace_for(w, bytes, s, &werr);
+    if (!ws.ptr) return werr;
     const dim3 grid(nm * nn * splits);
     if (p.fmt == 1)
-      run_ilv8<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, 1, 1>(p, s, grid, ws, splits);
+      run_ilv8<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, 1, 1>(p, s, grid, ws.ptr, splits);
     else
-      run_ilv8<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, 2, 1>(p, s, grid, ws, splits);
+      run_ilv8<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, 2, 1>(p, s, grid, ws.ptr, splits);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_reduce(ws, splits, p.M, p.N, p.C, p.ldc, s);
+    return launch_reduce(ws.ptr, splits, p.M, p.N, p.C, p.ldc, s);
   }
   return hipErrorInvalidConfiguration;  // not reached: splits == 1 where SW == 0
 }
@@ -199,13 +199,13 @@ hipError_t launch_ilv8_planned(const W8A16Params& p, hipStream_t s, const Worksp
     *w.need = bytes;
     return hipSuccess;
   }
-  float* ws = nullptr;
+  Lease ws;
   if (bytes) {
     hipError_t err = hipSuccess;
     ws = workspace_for(w, bytes, s, &err);
-    if (!ws) pl = ilv8_plan<BNO>(p, cols, false, &tail);  // no workspace: unsplit
+    if (!ws.ptr) pl = ilv8_plan<BNO>(p, cols, false, &tail);  // no workspace: unsplit
   }
-  if (!tail) return run_plan<GROUP, XCD, RSP>(p, s, ws, pl, GU);
+  if (!tail) return run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, GU);
   if constexpr (GU)
     return launch_ilv8_gu_tail<256, 256, 64, 1, 4, 3, GROUP, XCD, RSP, 128, 128, 128, 1, 4, 2, 0, 0>(p, s, w);
   else
@@ -234,9 +234,12 @@ bool plan_instead(const W8A16Params& p, hipStream_t s, const Workspace& w, doubl
     *w.need = bytes;
     return true;
   }
-  float* ws = nullptr;
-  if (bytes && !(ws = workspace_for(w, bytes, s, e))) return false;
-  *e = run_plan<GROUP, XCD, RSP>(p, s, ws, pl, false);
+  Lease ws;
+  if (bytes) {
+    ws = workspace_for(w, bytes, s, e);
+    if (!ws.ptr) return false;
+  }
+  *e = run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, false);
   return true;
 }
 
