@@ -81,6 +81,9 @@ tempo::gen8::W8A16Params to_pod(const TempoW8A16Params* p) {
 // device with hipGetSymbolAddress, with that device current, and kept in scratch_ptr[].
 static __device__ __align__(256) unsigned char scratch[TEMPO_NOALLOC_SCRATCH_BYTES];
 
+static_assert(tempo::gen8::kPlanWorkspace <= TEMPO_NOALLOC_SCRATCH_BYTES,
+              "a plan's partial sums fit the static array");
+
 constexpr int kMaxDevices = 64;
 void* scratch_ptr[kMaxDevices] = {};
 std::mutex scratch_mu;
@@ -176,6 +179,7 @@ int tempo_gemm_w8a16_launch_noalloc(const TempoW8A16Params* p, tempo_stream_t st
   w.ptr = device_scratch(&err);
   if (!w.ptr) return (int)err;
   w.bytes = TEMPO_NOALLOC_SCRATCH_BYTES;
+  w.shared = true;
   w.pool = false;  // a row whose workspace exceeds the scratch returns hipErrorOutOfMemory
   return (int)tempo::gen8::launch_with(to_pod(p), static_cast<hipStream_t>(stream), w);
 }

@@ -17,6 +17,15 @@
  *     streams never share a workspace, and threads may call on one stream at once: a call holds
  *     the buffer's lock until its last kernel is enqueued.  Every other row uses no workspace and
  *     allocates nothing.
+ *   - some rows only gain by a workspace (plans that split K, the sliced decode kernel in place of
+ *     an unsliced row): without one they run unsplit, as fast as they can and with their fp32 sums
+ *     in another order.  They take the caller's memory, and the pool except where work on another
+ *     stream may come to use the same buffer: on a stream under graph capture and on
+ *     hipStreamPerThread.  tempo_gemm_*_workspace_bytes counts them.
+ *   - a graph captured over the pool (the rows that cannot do without, on a stream whose buffer is
+ *     large enough) holds that buffer: replay it on that stream only, or capture the *_launch_ws
+ *     entries.  The same rows share one buffer between all threads' hipStreamPerThread streams:
+ *     hand over a workspace there.
  *   - the int returned is a hipError_t value: 0 = success; TEMPO_FALLBACK (9, the value of
  *     hipErrorInvalidConfiguration) = "shape not covered, take your own path" -- a legal
  *     answer, not a failure (reference kernels/shipped/gemm_fp16/sm_70/dispatch.inc:12-13,26).
@@ -60,16 +69,16 @@ int tempo_gemm_fp16_applicable(const TempoGemmParams* p);
  * stream), allocated on first use and grown with hipMalloc when a larger shape needs it (a
  * grown-out buffer is kept, not freed, until the process ends, so work already queued or a graph
  * captured earlier never sees it freed).  On a stream under graph capture the pool cannot grow:
- * such a call returns hipErrorStreamCaptureUnsupported (900) and launches nothing; use
- * tempo_gemm_fp16_launch_ws there. */
+ * a row that cannot do without returns hipErrorStreamCaptureUnsupported (900) there and launches
+ * nothing, and one that can runs unsplit; use tempo_gemm_fp16_launch_ws there. */
 int tempo_gemm_fp16_launch(const TempoGemmParams* p, tempo_stream_t stream);
 /* tempo_gemm_fp16_launch with the caller's workspace (ws, ws_bytes device memory; may be NULL /
- * 0 for shapes whose row needs none): never allocates, never synchronises.  A row needing more
- * than ws_bytes (tempo_gemm_fp16_workspace_bytes) returns hipErrorOutOfMemory (2) without
- * launching -- at M <= 128 (fp16: 256); rows above that split K only where they are given the
- * workspace and run unsplit otherwise, here and on a stream under capture.  No reference counterpart (its launcher has no workspace, launch.cuh:20-26): this
- * is for callers whose own allocator must own every buffer -- a framework capturing HIP graphs
- * (torch's graph-aware caching allocator), arenas of a serving loop. */
+ * 0 for shapes whose row needs none): never allocates, never synchronises.  With less than
+ * tempo_gemm_fp16_workspace_bytes a row that can do without runs unsplit; one that cannot
+ * returns hipErrorOutOfMemory (2) without launching where ws_bytes is less than its own splits
+ * need.  No reference counterpart (its launcher has no workspace, launch.cuh:20-26): this is for
+ * callers whose own allocator must own every buffer -- a framework capturing HIP graphs (torch's
+ * graph-aware caching allocator), arenas of a serving loop. */
 int tempo_gemm_fp16_launch_ws(const TempoGemmParams* p, void* ws, size_t ws_bytes,
                               tempo_stream_t stream);
 /* Bytes of workspace the row tempo_gemm_fp16_launch runs for this shape needs (0: none, or not
@@ -116,18 +125,19 @@ size_t tempo_gemm_w8a16_workspace_bytes(const TempoW8A16Params* p);
 
 /* tempo_gemm_w8a16_launch that allocates nothing, for callers that cannot allocate (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in
- * the reference.  Same rows, kernels and results as tempo_gemm_w8a16_launch (bit for bit); a
- * split-K row takes its workspace from a static device array of TEMPO_NOALLOC_SCRATCH_BYTES per
- * GPU instead of the allocating pool, and a row that would need more returns
- * hipErrorOutOfMemory (2) without launching.  The current ladder never needs more: an
- * interleaved split-K row keeps tiles x splits <= 256, so its workspace is at most
- * 256 x 128 x 256 x 4 bytes = 32 MiB; a line row with k slices needs ks x M x N x 4 bytes with
- * ks <= 8 and M <= 32, and slices only grids short of whole rounds of the part (3.75 MiB at most
- * today, at (32, 5120, 12288)).
- * Every call on one GPU shares that GPU's array (the first call on a device looks its address
- * up): calls that overlap on one GPU -- on different streams, or from different threads without
- * ordering -- race on it.  Nothing in it needs clearing: a split-K launch writes every partial
- * sum it later reads. */
+ * the reference.  A row that cannot run without a workspace takes it from a static device array of
+ * TEMPO_NOALLOC_SCRATCH_BYTES per GPU instead of the allocating pool, with the kernels and
+ * results of tempo_gemm_w8a16_launch (bit for bit); a row that only gains by one runs unsplit
+ * (its fp32 sums in another order), so such calls share nothing.  A row that would need more than
+ * the array returns hipErrorOutOfMemory (2) without launching; the current ladder never does.  An
+ * interleaved split-K row keeps tiles x splits <= 256, at most 256 x 128 x 256 x 4 bytes =
+ * 32 MiB; a plan that runs in its place keeps its partial sums within 32 MiB; a line row with k
+ * slices, or the sliced kernel in its place, needs ks x M x N x 4 bytes with ks <= 8 and M <= 32
+ * (11.9 MiB at most over N up to 40000 and K up to 65536, at (32, 12160, 12288)).
+ * Every call that takes the array shares it with the others on its GPU (the first call on a device
+ * looks its address up): such calls must not overlap on one GPU -- on different streams, or from
+ * different threads without ordering.  Nothing in it needs clearing: a split-K launch writes every
+ * partial sum it later reads. */
 #define TEMPO_NOALLOC_SCRATCH_BYTES (32u << 20)
 int tempo_gemm_w8a16_launch_noalloc(const TempoW8A16Params* p, tempo_stream_t stream);
 

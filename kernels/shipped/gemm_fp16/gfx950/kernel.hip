@@ -2442,13 +2442,14 @@ __global__ __launch_bounds__(TPB) void k_stream_line(StreamArgs p, int G) {
 // between them.
 
 // Workspace of a split-K row.  `ptr`/`bytes`: device memory the caller hands over (may be
-// null / 0); `pool`: the row may take the delivery's per-(device, stream) pool instead; `need`:
-// when set, the row only reports the bytes it needs (0 for rows without a workspace) and
-// launches nothing.
+// null / 0), `shared` where calls on other streams take the same memory; `pool`: the row may take
+// the delivery's per-(device, stream) pool instead; `need`: when set, the row only reports the
+// bytes it needs (0 for rows without a workspace) and launches nothing.
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
   bool pool = false;
+  bool shared = false;
   size_t* need = nullptr;
 };
 
@@ -2526,6 +2527,32 @@ inline Lease workspace_for(const Workspace& w, size_t bytes, hipStream_t s, hipE
   else
     *err = hipErrorOutOfMemory;
   return l;
+}
+
+// The workspace of a split that a row only gains by: its own path needs `own` bytes.  Where that is
+// none, the call takes no memory that work on another stream may be using -- a `shared` workspace,
+// the pool of a stream under capture (its graph may be replayed on any stream), the pool under
+// hipStreamPerThread (one handle, a stream per thread) -- so that calls which need nothing share
+// nothing.
+inline Lease workspace_to_gain(const Workspace& w, size_t bytes, size_t own, hipStream_t s,
+                               hipError_t* err) {
+  if (own == 0) {
+    const bool given = w.ptr && w.bytes >= bytes;
+    bool refuse = given ? w.shared : w.pool && s == hipStreamPerThread;
+    if (!given && w.pool && !refuse) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+        (void)hipGetLastError();  // the caller goes on without a workspace
+        refuse = true;
+      }
+      refuse = refuse || cs != hipStreamCaptureStatusNone;
+    }
+    if (refuse) {
+      *err = hipErrorOutOfMemory;
+      return Lease{};
+    }
+  }
+  return workspace_for(w, bytes, s, err);
 }
 
 // Split count of a split-K row: the most splits such that tiles x splits stays within `slots`

@@ -297,11 +297,12 @@ inline constexpr PlanTable kPlanTables[] = {
 #include "plan.inc"
 };
 #undef TEMPO_TABLE
-// The plan in place of a row whose own time is estimated at own_us: true (with *e) where the plan is
-// below `ahead` of it, the interleaved kernel takes the shape and the plan's workspace can be had.
+// The plan in place of a row whose own time is estimated at own_us and which needs own_bytes of
+// workspace: true (with *e) where the plan is below `ahead` of it, the interleaved kernel takes the
+// shape and the plan's workspace can be had (workspace_to_gain).
 template <int GROUP, int XCD, int RSP>
 bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double own_us,
-                  double ahead, hipError_t* e);
+                  double ahead, size_t own_bytes, hipError_t* e);
 
 // One dispatch row: launchers without a workspace ignore it (and, asked for their need, report 0).
 inline hipError_t call_row(hipError_t (*f)(const GemmParams&, hipStream_t), const GemmParams& p,
@@ -323,7 +324,7 @@ template <int BM, int BN, int BK, int WM, int WN, int STAGES, int SWZ, int GROUP
 inline hipError_t launch_dma_or_plan(const GemmParams& p, hipStream_t s, const Workspace& w) {
   hipError_t e = hipSuccess;
   const double own = tile_us(plan_table(kPlanTables, p.M), RATE100 * 0.01, BM, BN, BK, p.M, p.N, p.K, 1);
-  if (plan_instead<8, 1, 8>(p, s, w, own, p.M <= 128 ? 0.85 : 0.95, &e)) return e;
+  if (plan_instead<8, 1, 8>(p, s, w, own, p.M <= 128 ? 0.85 : 0.95, 0, &e)) return e;
   if (w.need) {
     *w.need = 0;
     return hipSuccess;
@@ -335,8 +336,8 @@ inline hipError_t launch_dma_or_plan(const GemmParams& p, hipStream_t s, const W
 // the activations (at M <= 16 half of the padding too), at 9.7 (M <= 16) or 10.5 TB/s over the part
 // in whole rounds of groups over the CUs; a k-slice row's second kernel 5.  Within 15 % of M = 4 ..
 // 32, N = 2560 .. 11008, K = 2560 .. 17408; too low past M = 32, where the plan wins by far more.
-inline double line_us(const GemmParams& p, int mb, int sn, int KS) {
-  const int wgs = p.N / (16 * sn), ks = KS > 1 ? line_kslices(wgs, p.K, KS) : 1;
+inline double line_us(const GemmParams& p, int mb, int sn, int ks) {
+  const int wgs = p.N / (16 * sn);
   const long w = (long)wgs * ks;
   const int rows = 16 * sn + (mb == 1 ? (16 + p.M) / 2 : p.M);
   const double mbytes = (double)wgs * p.K * 2e-6 * rows;
@@ -350,7 +351,9 @@ inline hipError_t launch_line_or_plan(const GemmParams& p, hipStream_t s, const 
   // weight rows a multiple of 16 KiB apart: a tile's 128 rows fall on few HBM channels ((16, 8192,
   // 8192): 36 us planned, 32 on the row)
   const bool aliased = p.M <= 32 && p.ldb % 8192 == 0;
-  if (!aliased && plan_instead<8, 1, 8>(p, s, w, line_us(p, MB, SN, KS), 0.88, &e)) return e;
+  const int ks = KS > 1 ? line_kslices(p.N / (16 * R * SN), p.K, KS) : 1;
+  const size_t own = ks > 1 ? (size_t)ks * p.M * p.N * sizeof(float) : 0;
+  if (!aliased && plan_instead<8, 1, 8>(p, s, w, line_us(p, MB, SN, ks), 0.88, own, &e)) return e;
   if constexpr (KS > 1) {
     return launch_line_ks<MB, R, D, SN, WAVES, KS>(p, s, w);
   } else {

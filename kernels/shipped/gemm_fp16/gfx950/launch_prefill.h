@@ -135,7 +135,7 @@ hipError_t launch_ilv_planned(const GemmParams& p, hipStream_t s, const Workspac
   Lease ws;
   if (bytes) {
     hipError_t err = hipSuccess;
-    ws = workspace_for(w, bytes, s, &err);
+    ws = workspace_to_gain(w, bytes, 0, s, &err);
     if (!ws.ptr) pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, false);  // unsplit
   }
   return run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, gate_up);
@@ -148,7 +148,7 @@ hipError_t launch_ilv_plan(const GemmParams& p, hipStream_t s, const Workspace& 
 
 template <int GROUP, int XCD, int RSP>
 bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double own_us,
-                  double ahead, hipError_t* e) {
+                  double ahead, size_t own_bytes, hipError_t* e) {
   constexpr int kLd = 0x7fffffff / (2 * 256);
   if (p.lda > kLd || p.ldb > kLd) return false;
   const TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, p.N, p.K, true);
@@ -161,7 +161,7 @@ bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double
   }
   Lease ws;
   if (bytes) {
-    ws = workspace_for(w, bytes, s, e);
+    ws = workspace_to_gain(w, bytes, own_bytes, s, e);
     if (!ws.ptr) return false;
   }
   *e = run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, false);
@@ -175,7 +175,9 @@ hipError_t launch_ilv_or_plan(const GemmParams& p, hipStream_t s, const Workspac
   hipError_t e = hipSuccess;
   if (plan_instead<GROUP, XCD, RSP>(p, s, w,
                                     tile_us(plan_table(kPlanTables, p.M), RATE100 * 0.01, BM, BN, BK,
-                                            p.M, p.N, p.K, splits), 0.95, &e))
+                                            p.M, p.N, p.K, splits), 0.95,
+                                    splits > 1 ? (size_t)splits * p.M * p.N * sizeof(float) : 0,
+                                    &e))
     return e;
   return launch_ilv<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, SW, MINKT>(p, s, w);
 }

@@ -536,11 +536,12 @@ template <int GROUP, int XCD, int RSP>
 hipError_t launch_ilv8_plan(const W8A16Params& p, hipStream_t s, const Workspace& w);
 template <int GROUP, int XCD, int RSP>
 hipError_t launch_ilv8_plan_gu(const W8A16Params& p, hipStream_t s, const Workspace& w);
-// The plan in place of a row whose own time is estimated at own_us: true (with *e) where the plan is
-// 5 % ahead, the interleaved kernel takes the shape and the plan's workspace can be had.
+// The plan in place of a row whose own time is estimated at own_us and which needs own_bytes of
+// workspace: true (with *e) where the plan is 5 % ahead, the interleaved kernel takes the shape and
+// the plan's workspace can be had (workspace_to_gain).
 template <int GROUP, int XCD, int RSP>
 bool plan_instead(const W8A16Params& p, hipStream_t s, const Workspace& w, double own_us,
-                  hipError_t* e);
+                  size_t own_bytes, hipError_t* e);
 // A split-K row of its own, or the plan where that is ahead (R..: its rates in 1/100, unsplit and
 // split, int8 and uint8).
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP,
@@ -597,7 +598,7 @@ inline bool phase_instead(const W8A16Params& p, hipStream_t s, const Workspace& 
     *w.need = std::max(bytes, own_bytes);
     return true;
   }
-  const Lease lease = workspace_for(w, bytes, s, e);
+  const Lease lease = workspace_to_gain(w, bytes, own_bytes, s, e);
   if (!lease.ptr) return false;
   Workspace ws;
   ws.ptr = lease.ptr;
@@ -698,7 +699,7 @@ inline hipError_t launch_line_or_plan(const W8A16Params& p, hipStream_t s, const
   hipError_t e = hipSuccess;
   const double own = tile_us(plan_table(kPlanTables, p.M), 0.01 * (p.fmt == 1 ? R1 : R2), 16 * MB,
                              16 * R * SN, 128, p.M, p.N, p.K, 1);
-  if (plan_instead<8, 1, 8>(p, s, w, own, &e)) return e;
+  if (plan_instead<8, 1, 8>(p, s, w, own, 0, &e)) return e;
   if (w.need) {
     *w.need = 0;
     return hipSuccess;

@@ -202,7 +202,7 @@ hipError_t launch_ilv8_planned(const W8A16Params& p, hipStream_t s, const Worksp
   Lease ws;
   if (bytes) {
     hipError_t err = hipSuccess;
-    ws = workspace_for(w, bytes, s, &err);
+    ws = workspace_to_gain(w, bytes, 0, s, &err);
     if (!ws.ptr) pl = ilv8_plan<BNO>(p, cols, false, &tail);  // no workspace: unsplit
   }
   if (!tail) return run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, GU);
@@ -223,7 +223,7 @@ hipError_t launch_ilv8_plan_gu(const W8A16Params& p, hipStream_t s, const Worksp
 
 template <int GROUP, int XCD, int RSP>
 bool plan_instead(const W8A16Params& p, hipStream_t s, const Workspace& w, double own_us,
-                  hipError_t* e) {
+                  size_t own_bytes, hipError_t* e) {
   constexpr int kLd = 0x7fffffff / (2 * 256);
   if (p.lda > kLd || p.ldw > kLd) return false;
   const TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, p.fmt - 1, p.M, p.N, p.K, true);
@@ -236,7 +236,7 @@ bool plan_instead(const W8A16Params& p, hipStream_t s, const Workspace& w, doubl
   }
   Lease ws;
   if (bytes) {
-    ws = workspace_for(w, bytes, s, e);
+    ws = workspace_to_gain(w, bytes, own_bytes, s, e);
     if (!ws.ptr) return false;
   }
   *e = run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, false);
@@ -251,7 +251,9 @@ hipError_t launch_ilv8_or_plan(const W8A16Params& p, hipStream_t s, const Worksp
   hipError_t e = hipSuccess;
   if (plan_instead<GROUP, XCD, RSP>(p, s, w,
                                     tile_us(plan_table(kPlanTables, p.M), 0.01 * rate, BM, BN, BK,
-                                            p.M, p.N, p.K, splits), &e))
+                                            p.M, p.N, p.K, splits),
+                                    splits > 1 ? (size_t)splits * p.M * p.N * sizeof(float) : 0,
+                                    &e))
     return e;
   return launch_ilv8<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, SW, MINKT>(p, s, w);
 }
