@@ -5,10 +5,12 @@ runtime's entry points in a process of its own, and each call's kernels come bac
 
 A call: op 0 = gemm_fp16, 1 / 2 = gemm_w8a16 (formats 1, 2), 3..5 their fused gate/up forms; M, N, K;
 optional `entry` ("pool" (default), "ws", "none", "noalloc"; "none" is "ws" without a workspace),
-`stream` (a handle value), `capture` (true: that stream is under capture), `pads` (elements added to
-lda, ldb / ldw, ldc), `odd` (bytes added to the scale pointer).  A launch: dict(kernel, args,
-grid, block, stream, thread, first): `kernel` and the list of integer template arguments from the
-device symbol, `first` the first kernel argument (a split-K reduction's workspace address).
+`ws_bytes` (in place of what the shape asks for), `stream` (a handle value), `capture` (true: that
+stream is under capture), `pads` (elements added to lda, ldb / ldw, ldc), `odd` (bytes added to the
+scale pointer).  Or an attention call: fmha=[B, Sq, Sk, H, Hkv, D, causal], entry "ws" (default) or
+"none".  A launch: dict(kernel, args, grid, block, stream, thread, first): `kernel` and the list of
+integer template arguments from the device symbol, `first` the first kernel argument (a split-K
+reduction's workspace address).
 """
 import ctypes as ct
 import json
@@ -48,7 +50,19 @@ def _child_load(shim):
     return rec, capi, capi.lib()
 
 
+def _child_fmha(capi, L, c):
+    B, Sq, Sk, H, Hkv, D, causal = c["fmha"]
+    f = 0x100000
+    p = capi.TempoFmhaParams(f, f, f, f, None, B, H, Hkv, Sq, Sk, D, 0.1, int(causal),
+                             Sq * H * D, H * D, D, Sk * Hkv * D, Hkv * D, D,
+                             Sk * Hkv * D, Hkv * D, D, Sq * H * D, H * D, D)
+    need = L.tempo_fmha_fwd_workspace_bytes(p) if c.get("entry", "ws") == "ws" else 0
+    return L.tempo_fmha_fwd_launch_ws(p, WS if need else None, need, 0x50)
+
+
 def _child_call(capi, L, c):
+    if "fmha" in c:
+        return _child_fmha(capi, L, c)
     op, M, N, K = c["op"], c["M"], c["N"], c["K"]
     base, gu = op % 3, op >= 3
     pa, pb, pc = c.get("pads", (0, 0, 0))
@@ -65,6 +79,7 @@ def _child_call(capi, L, c):
     if entry == "noalloc":
         return getattr(L, name + "_launch_noalloc")(p, s)
     need = getattr(L, name + "_workspace_bytes")(p) if entry == "ws" else 0
+    need = c.get("ws_bytes", need)
     return getattr(L, name + "_launch_ws")(p, WS if need else None, need, s)
 
 
@@ -151,6 +166,28 @@ def record(calls):
 def record_threads(calls, repeat=20, delay_us=500):
     """The launches of one thread per call, each making its call `repeat` times."""
     return _run(dict(mode="threads", calls=calls, repeat=repeat, delay_us=delay_us))
+
+
+def own_kernel(row, fmt, gu):
+    """(kernel, leading template arguments) of a row's own kernel."""
+    kind, p = row[3], row[4]
+    epi = int(gu)
+    if kind in ("ilv", "ilv8", "dma", "mfma"):
+        name = {"ilv": "k_gemm_ilv", "ilv8": "k_gemm_ilv8", "dma": "k_gemm_dma",
+                "mfma": "k_gemm"}[kind]
+        return name, [p[k] for k in ("BM", "BN", "BK", "WM", "WN")] + (
+            [p["STAGES"]] if kind != "mfma" else [])
+    if kind == "line":
+        tpb = 512 if p["MB"] >= 4 else 1024
+        if p.get("MT"):
+            return "k_stream_line", [p["MB"], p["R"], p["D"], fmt, 0, 1, 64 * p["S"], 0]
+        return "k_stream_line", [p["MB"], p["R"], p["D"], fmt, epi, p.get("SN", 1), tpb,
+                                 p.get("TL", 0)]
+    if kind == "phase":
+        return "k_stream_phase", [p["MB"], p["NS"], p["D"], fmt, epi, int(p.get("KS", 1) > 1)]
+    if kind == "stream":
+        return "k_stream", [p["MB"], p["R"], p["U"], fmt]
+    return "k_stream_sh", [p["MB"], p["R"], p["U"], fmt, p["SN"]]
 
 
 if __name__ == "__main__":

@@ -1,5 +1,5 @@
-"""PLAN rows (tile and split count by an estimate of the time): select.py's plan and the compiled one
-agree over a sweep, and the GPU results meet the oracle where a plan changes: one split and many, the
+"""PLAN rows (tile and split count by an estimate of the time): what the rule says -- plan or the row's
+own kernel, which tile, how many splits -- and what the library launches agree over a sweep, and the GPU results meet the oracle where a plan changes: one split and many, the
 last split shorter, ragged M against every tile height, N in one 128-column tile, and without a
 workspace.
 
@@ -15,6 +15,7 @@ import pytest
 
 from cuda_tempiler_amd import capi
 from oracle import oracle as O
+from tests.launch_recorder import own_kernel, record
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -51,55 +52,122 @@ def _own(row, M, N, K):
     return -(-kt // -(-kt // sp)) if sp > 1 else 1
 
 
-def _check(fmt, row, M, N, K, plan):
-    """The compiled need is the plan's, or, where a row of its own competes, that row's."""
-    us, _, sp, tail = plan
-    need = capi.workspace_bytes(fmt, M, N, K)
-    unit = M * N * 4
-    want = 0 if tail or sp == 1 else sp * unit
-    own = _own(row, M, N, K)
-    if own and "RATE" in row:
+def _kslices(wgs, K, KS):
+    """line_kslices of launch.h."""
+    steps, best = K // 128, 1
+
+    def even(ks):
+        return wgs * ks / (-(-wgs * ks // 256) * 256)
+
+    for ks in range(2, KS + 1):
+        if steps % ks == 0 and steps // ks >= 8 and even(ks) > even(best) + 1e-9:
+            best = ks
+    return best if even(best) >= even(1) + 0.08 else 1
+
+
+def _line_us(M, N, K, p):
+    """line_us of the fp16 launch.h."""
+    sn = p.get("SN", 1)
+    wgs = N // (16 * sn)
+    ks = _kslices(wgs, K, p["KS"]) if p.get("KS", 1) > 1 else 1
+    rows = 16 * sn + ((16 + M) // 2 if p["MB"] == 1 else M)
+    w = wgs * ks
+    return 3 + (0.103 if p["MB"] == 1 else 0.095) * wgs * K * 2e-6 * rows * (
+        -(-w // 256) * 256) / w + (5 if ks > 1 else 0)
+
+
+def _choice(op, row, M, N, K):
+    """What a row with a plan runs, given a workspace: (index into PLAN_TILES, splits), "tail", or
+    "own"."""
+    sel, f = (F16, 0) if op == 0 else (W8, op - 1)
+    kind = row["kind"]
+    if op and kind == "mfma" and K % 128:
+        return "own"
+    if kind in ("ilv8", "mfma") and "RATE" not in row:
+        _, tile, sp, tail = W8.plan(M, N, K, op)
+        return "tail" if tail else (tile, sp)
+    plan = sel.plan_tiles(M, N, K, f)
+    if kind == "ilv" and not row.get("SW"):
+        return plan[1:]
+    if plan is None:
+        return "own"
+    if kind == "line" and op == 0:
+        own, ahead = _line_us(M, N, K, row), 0.88
+        if M <= 32 and K % 8192 == 0:
+            return "own"
+    else:
+        if kind == "line":
+            bm, bn, bk = 16 * row["MB"], 16 * row["R"] * row.get("SN", 1), 128
+        else:
+            bm, bn, bk = row["BM"], row["BN"], row["BK"]
+        sp = _own(row, M, N, K) or 1
         rates = row["RATE"] if isinstance(row["RATE"], tuple) else (row["RATE"],)
-        rates = row.get("RATES", rates) if own > 1 else rates
-        sel = F16 if fmt == 0 else W8
-        if us >= 0.95 * sel.tile_us(M, N, K, row["BM"], row["BN"], row["BK"], rates[max(fmt - 1, 0)],
-                                    own):
-            want = 0 if own == 1 else own * unit
-    elif row["kind"] in ("line", "dma"):  # the plan or the row (whose k slices are its own affair)
-        assert need == want or need in (0, 2 * unit, 4 * unit, 8 * unit), (fmt, M, N, K)
-        return need == want and sp > 1
-    assert need == want <= W8.PLAN_WS, (fmt, M, N, K, row["tag"])
-    return sp > 1
+        rates = row.get("RATES", rates) if sp > 1 else rates
+        own = sel.tile_us(M, N, K, bm, bn, bk, rates[f], sp)
+        ahead = 0.85 if kind == "dma" and M <= 128 else 0.95
+    return plan[1:] if plan[0] < ahead * own else "own"
+
+
+def _check(op, shapes):
+    """The library's launches against _choice; returns how often each kind of choice was met."""
+    sel = F16 if op == 0 else W8
+    select = (lambda M, N, K: F16.select("gemm", M, N, K)) if op == 0 else (
+        lambda M, N, K: W8.select("gemm_w8a16", M, N, K, fmt=op))
+    shapes = [(M, N, K, select(M, N, K)) for M, N, K in shapes]
+    shapes = [x for x in shapes if x[3] and x[3].get("PLAN")]
+    met = {}
+    for (M, N, K, row), got in zip(shapes, record([
+            dict(op=op, M=M, N=N, K=K, entry="ws") for M, N, K, _ in shapes])):
+        want = _choice(op, row, M, N, K)
+        what = (op, M, N, K, row["tag"], want, got)
+        assert got["rc"] == 0, what
+        names = [l["kernel"] for l in got["launches"]]
+        reduces = sum(n.startswith("k_splitk_reduce") for n in names)
+        first = got["launches"][0]
+        if want == "tail":
+            assert names == ["k_gemm_ilv8"] * 2 and first["args"][:2] == [256, 256], what
+            key = "tail"
+        elif want == "own":
+            full = (None, None, row["tag"], row["kind"], row)
+            name, args = own_kernel(full, op, False)
+            assert names[0] == name and first["args"][:len(args)] == args, what
+            key = "own " + row["kind"]
+        else:
+            tile, sp = want
+            bm, bn = sel.PLAN_TILES[tile][:2]
+            assert names[0] == ("k_gemm_ilv" if op == 0 else "k_gemm_ilv8"), what
+            assert tuple(first["args"][:6]) == sel.PLAN_TILES[tile][:6], what
+            assert first["grid"] == -(-M // bm) * (N // bn) * sp and reduces == (sp > 1), what
+            need = capi.workspace_bytes(op, M, N, K)
+            assert need == (0 if sp == 1 else sp * M * N * 4) <= W8.PLAN_WS, what
+            key = "split" if sp > 1 else "unsplit"
+        met[key] = met.get(key, 0) + 1
+    return met
 
 
 @pytest.mark.parametrize("fmt", [1, 2])
 def test_w8a16_plans_agree(fmt):
-    split = tails = 0
+    wide = [(M, N, K) for M in (33, 48, 64) for N in (12288, 15360, 17408) for K in (640, 5120)]
+    met = _check(fmt, SWEEP + wide + [(200, 3840, 3904), (256, 5120, 5184)])
+    own = {"own line", "own ilv8"} | ({"own mfma"} if fmt == 1 else set())  # fmt 2: whole 128 k
+    assert {"split", "unsplit", "tail"} | own <= set(met), met
     for M, N, K in SWEEP:
-        row = W8.select("gemm_w8a16", M, N, K, fmt=fmt)
-        if row and row.get("PLAN"):
-            plan = W8.plan(M, N, K, fmt)
-            split += _check(fmt, row, M, N, K, plan)
-            tails += plan[3]
         row = W8.select_gate_up("gemm_w8a16_gate_up", M, N, K, fmt=fmt)
         if row and row.get("PLAN"):
             _, _, sp, tail = W8.plan(M, N, K, fmt, gate_up=True)
             want = 0 if tail or sp == 1 else sp * M * 2 * N * 4
             assert _gate_up_need(fmt, M, N, K) == want <= W8.PLAN_WS, (M, N, K)
-    assert split and tails
 
 
 def test_fp16_plans_agree():
-    split = 0
-    for M, N, K in SWEEP + [(M, N, K) for M, N, K in SWEEP if M == 33 for M in (8, 17, 32)]:
-        row = F16.select("gemm", M, N, K)
-        if row and row.get("PLAN"):
-            split += _check(0, row, M, N, K, (F16.plan(M, N, K) or (0, 0, 1)) + (False,))
+    few = [(M, N, K) for _, N, K in SWEEP if _ == 33 for M in (2, 8, 16, 17, 24, 32, 48)]
+    met = _check(0, SWEEP + few + [(16, 4096, 8192), (32, 5120, 16384)])  # rows 16 KiB apart
+    assert {"split", "unsplit", "own line", "own dma", "own ilv"} <= set(met), met
+    for M, N, K in SWEEP:
         row = F16.select_gate_up("gemm_gate_up", M, N, K)
         if row and row.get("PLAN") and not (M > 128 and W8.tail_split(M, N, 256, 128)):
             _, _, sp = F16.plan(M, N, K, gate_up=True)
             assert _gate_up_need(0, M, N, K) == (0 if sp == 1 else sp * M * 2 * N * 4), (M, N, K)
-    assert split
 
 
 CASES = [  # M, N, K
