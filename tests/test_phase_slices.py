@@ -10,7 +10,8 @@ import pytest
 
 from cuda_tempiler_amd import capi
 from oracle import oracle as O
-from tests.test_plan_rows import _dev, _weights
+from tests.launch_recorder import record
+from tests.test_plan_rows import W8, _dev, _kslices, _weights
 
 SLICED = [  # M, N, K, slices
     (2, 2048, 8192, 8),     # 64 rows a workgroup: 4 slabs
@@ -19,13 +20,72 @@ SLICED = [  # M, N, K, slices
     (32, 5120, 5120, 4),    # 5 slabs
     (24, 3584, 18944, 4),   # 56 rows: a part slab, 37 steps
     (9, 10240, 5120, 4),    # 160 rows: 10 slabs
+    (16, 11264, 8192, 2),   # 88 rows: 6 slabs, 32 steps
+    (13, 10752, 13312, 2),  # 84 rows: a part slab
+    (31, 11264, 5120, 2),
+    (32, 10752, 5120, 2),
 ]
 EVEN = [(16, 8192, 8192), (16, 7168, 5120), (32, 5120, 4096)]  # the line grid fills its rounds
 
 
+def _slices(fmt, M, N, K):
+    """phase_slices of launch.h: (slices, slabs) of the k-sliced phase kernel, or None."""
+    mb = 1 if M <= 16 else 2
+    for ks in (4, 2, 8):
+        for ns in range(4, 11):
+            if W8.phase_fits(dict(MB=mb, NS=ns, D=4, KS=ks), M, N, K, fmt):
+                return ks, ns
+    return None
+
+
+def _choice(fmt, row, M, N, K):
+    """(slices, slabs) of the phase kernel where a row runs that, else None (launch_line_or_phase,
+    launch_phase_row)."""
+    cut = _slices(fmt, M, N, K)
+    if row["kind"] == "phase":
+        return cut if cut else (row["KS"], row["NS"])
+    if not cut:
+        return None
+    wgs = N // (16 * row["R"] * row["SN"])
+    own = _kslices(wgs, K, row["KS"]) if row.get("KS", 1) > 1 else 1
+    grid = wgs * own
+    idle = N * K / 7.2e6 * (-(-grid // 256) * 256 - grid) / grid
+    part = (own - cut[0]) * 2.0 * M * N * 4 / 2.5e6 if own > 1 else 0
+    return cut if idle + part > row["PHASE"] else None
+
+
+@pytest.mark.parametrize("fmt", [1, 2])
+def test_sliced_rows_agree(fmt):
+    """The rule above and what the library launches, over the rows that may be sliced."""
+    shapes = [(M, N, K) for M in (2, 9, 16, 17, 24, 32)
+              for N in (2048, 2560, 3072, 3584, 4096, 4736, 5120, 6144, 7168, 8192, 10240, 10752, 11264)
+              for K in (2048, 4096, 5120, 5248, 6144, 8192, 12288, 17408, 18944)]
+    rows = [(x, W8.select("gemm_w8a16", *x, fmt=fmt)) for x in shapes]
+    rows = [(x, r) for x, r in rows if r and r["kind"] in ("line", "phase")
+            and ("PHASE" in r or r.get("KS", 1) > 1 and r["kind"] == "phase") and not r.get("TL")]
+    met = {}
+    for (x, r), got in zip(rows, record([dict(op=fmt, M=M, N=N, K=K, entry="ws")
+                                         for (M, N, K), _ in rows])):
+        want = _choice(fmt, r, *x)
+        first, what = got["launches"][0], (fmt, x, r["tag"], want, got)
+        assert got["rc"] == 0, what
+        if want:
+            ks, ns = want
+            assert first["kernel"] == "k_stream_phase", what
+            assert first["args"] == [1 if x[0] <= 16 else 2, ns, 4, fmt, 0, 1], what
+            assert got["launches"][1]["args"] == [ks], what
+        else:
+            assert first["kernel"] == "k_stream_line", what
+        met[want and want[0]] = met.get(want and want[0], 0) + 1
+    assert set(met) == {None, 2, 4, 8}, met
+
+
 @pytest.mark.parametrize("fmt", [1, 2])
 def test_which_shapes_are_sliced(fmt):
-    for M, N, K, ks in SLICED:
+    got = record([dict(op=fmt, M=M, N=N, K=K, entry="ws") for M, N, K, _ in SLICED])
+    for (M, N, K, ks), g in zip(SLICED, got):
+        assert [l["kernel"] for l in g["launches"]] == ["k_stream_phase", "k_splitk_reduce"], (M, N, K)
+        assert g["launches"][1]["args"] == [ks], (M, N, K)
         assert capi.workspace_bytes(fmt, M, N, K) >= ks * M * N * 4, (M, N, K)
     for M, N, K in EVEN:
         assert capi.workspace_bytes(fmt, M, N, K) == 0, (M, N, K)
@@ -51,7 +111,9 @@ def test_sliced_against_oracle(gpu, fmt, case):
     odd.copy_(ds)
     assert odd.data_ptr() % 4 == 2
     runs = [("pool", ds, None), ("torch", ds, "torch"), ("odd scale", odd, "torch")]
-    if K < 6144 and M <= 32 or M <= 16:
+    row = W8.select("gemm_w8a16", M, N, K, fmt=fmt)
+    if row["kind"] == "line" and (row.get("KS", 1) == 1 or _kslices(
+            N // (16 * row["R"] * row["SN"]), K, row["KS"]) == 1):
         runs.append(("none", ds, torch.empty(0, dtype=torch.uint8, device=gpu)))
     for what, sc, ws in runs:
         say("fmt", fmt, "case", case, what)
