@@ -190,3 +190,117 @@ def test_w8a16_gate_up_row_strided(gpu, fmt, case):
     full = host(Cw)
     assert O.count_poison(full[:, N:]) == full[:, N:].size, "padding columns written"
     _check(np.ascontiguousarray(full[:, :N]), O.gemm_gate_up_w8a16(A, q, s, z, 128, fmt), tag)
+
+
+@pytest.mark.parametrize("case", LC.FP16_GATE_UP_STRIDED, ids=LC.case_id)
+def test_fp16_gate_up_row_strided(gpu, case):
+    import torch
+    from cuda_tempiler_amd import capi
+
+    tag, M, N, K, pa, pb, pc = case
+    say("fp16 gate_up strided row", tag, "M", M, "N", N, "K", K, "pads", pa, pb, pc)
+    assert capi.route(3, M, N, K) == tag
+    A = O.randn_f16((M, K), 7 + M, 1.0)
+    B = O.randn_f16((2 * N, K), 13 + N, 2 * K ** -0.5)
+    dA, dB, _, _, Cw, dC = _strided_w8(gpu, A, B, A, None, M, N, K, pa, pb, pc)
+    capi.gemm_fp16_gate_up(dA, dB, C=dC)
+    torch.cuda.synchronize()
+    full = host(Cw)
+    assert O.count_poison(full[:, N:]) == full[:, N:].size, "padding columns written"
+    _check(np.ascontiguousarray(full[:, :N]), O.gemm_gate_up_f16(A, B), tag)
+
+
+@pytest.mark.parametrize("name,case", [(n, c) for n in sorted(LC.WITHOUT_PLAN)
+                                       for c in LC.WITHOUT_PLAN[n]],
+                         ids=lambda v: v if isinstance(v, str) else LC.case_id(v))
+def test_row_without_its_plan(gpu, name, case):
+    """The row's own kernel, where its plan's workspace is not there or lda is past the planned
+    tiles' offsets: the workspace is that of the row's own splits."""
+    import torch
+    from cuda_tempiler_amd import capi
+    from tests.test_ladder_coverage import LADDERS
+    from tests.test_ladder_kernels import _own_bytes
+
+    tag, M, N, K, pa = case
+    op = ["fp16", "w8_fmt1", "w8_fmt2"].index(name)
+    row = next(r for r in LADDERS[name][0] if r[2] == tag)
+    ws = torch.empty(_own_bytes(row, case), dtype=torch.uint8, device=gpu)
+    say(name, "row", tag, "M", M, "N", N, "K", K, "lda pad", pa, "workspace", ws.numel())
+    assert capi.route(op, M, N, K) == tag
+    A = O.randn_f16((M, K), 11 + M, K ** -0.5)
+    dA = dev(A, gpu)
+    if pa:
+        wide = torch.zeros((M, K + pa), dtype=torch.float16, device=gpu)
+        wide[:, :K] = dA
+        dA = wide[:, :K]
+    C = poisoned((M, N), gpu)
+    if op == 0:
+        B = O.randn_f16((N, K), 77 + N, K ** -0.5)
+        capi.gemm_fp16(dA, dev(B, gpu), C, workspace=ws)
+        ref = O.gemm_f16(A, B)
+    else:
+        q, s, z = _weights(N, K, op, 77 + N)
+        capi.gemm_w8a16(dA, dev(q, gpu), dev(s, gpu), dev(z, gpu) if z is not None else None,
+                        fmt=op, C=C, workspace=ws)
+        ref = O.gemm_w8a16(A, q, s, z, 128, op)
+    torch.cuda.synchronize()
+    _check(host(C), ref, tag)
+
+
+SPECIAL = [  # op, M, N, K: planned 64- and 128-row tiles with splits, sliced phase kernel, k slices
+    (0, 9, 5120, 5120), (0, 200, 7168, 5120), (1, 15, 5120, 17408), (2, 15, 11264, 13312),
+    (2, 50, 2560, 2560), (1, 300, 2560, 2560), (0, 5, 3840, 12288), (3, 100, 2048, 2048),
+    (5, 300, 1280, 4096),
+]
+
+
+@pytest.mark.parametrize("case", SPECIAL, ids=lambda c: "op%d-m%d-n%d-k%d" % c)
+def test_special_values_stay_in_their_row(gpu, case):
+    """An infinity and a NaN in two rows of A, and the lowest and largest fp16 value in a third:
+    their own rows of C are infinite or NaN where the exact product is (with the infinity's sign),
+    and every other row has the bits it has without them -- the rows past M that a tile pads with
+    included."""
+    import torch
+    from cuda_tempiler_amd import capi
+
+    op, M, N, K = case
+    fmt, gu = op % 3, op >= 3
+    rows = 2 * N if gu else N
+    A = dev(O.randn_f16((M, K), 5, K ** -0.5), gpu)
+    if fmt == 0:
+        B = dev(O.randn_f16((rows, K), 6, 1.0), gpu)
+        W = B.double()
+        run = lambda x: (capi.gemm_fp16_gate_up if gu else capi.gemm_fp16)(x, B)  # noqa: E731
+    else:
+        q, s, z = _weights(rows, K, fmt, 7)
+        dq, ds, dz = dev(q, gpu), dev(s, gpu), dev(z, gpu) if z is not None else None
+        f = capi.gemm_w8a16_gate_up if gu else capi.gemm_w8a16
+        run = lambda x: f(x, dq, ds, dz, fmt=fmt)  # noqa: E731
+        if fmt == 1:
+            W = (dq.double() * ds.double()[:, None]).half().double()
+        else:
+            W = ((dq.view(rows, -1, 128).double() - dz.double()[:, :, None])
+                 * ds.double()[:, :, None]).half().double().view(rows, K)
+    say("special values", case)
+    want = run(A).clone()
+    x = A.clone()
+    x[1, K // 2 + 3] = float("inf")
+    x[3, K - 1] = float("nan")
+    x[M - 1, 0], x[M - 1, K - 1] = -65504.0, 65504.0
+    got = run(x)
+    torch.cuda.synchronize()
+    rest = [i for i in range(M) if i not in (1, 3, M - 1)]
+    assert torch.equal(got[rest], want[rest])
+    assert torch.isnan(got[3]).all()
+    if gu:  # silu of an infinity is the epilogue's own affair
+        assert not torch.isfinite(got[1]).any()
+        return
+    y = (x[[1, M - 1]].double() @ W.t()).half()
+    assert torch.equal(torch.isnan(got[1]), torch.isnan(y[0]))
+    inf = torch.isinf(y[0])
+    assert torch.equal(torch.isinf(got[1]), inf) and torch.equal(got[1][inf], y[0][inf])
+    # the last row: +-65504 times two weights beside a sum of order 1; fp32 sums of K terms
+    big, ref = got[M - 1].double(), y[1].double()
+    ok = torch.isfinite(ref) & (ref.abs() < 6e4)
+    assert float((big - ref)[ok].norm()) <= 2e-3 * float(ref[ok].norm())
+    assert not torch.isnan(big[ok]).any()
