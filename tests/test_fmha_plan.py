@@ -22,6 +22,20 @@ def test_calls_without_a_workspace(B, Sq, Sk, H, Hkv, D):
     assert _need(B, Sq, Sk, H, Hkv, D) == 0
 
 
+def test_strided_gpu_cases_reach_every_form():
+    """The GPU cases on strided operands run the kernel they are listed with, cut where they say."""
+    from tests.launch_recorder import record
+    from tests.test_gpu_fmha_ranges import STRIDED
+
+    met = set()
+    for (case, kernel, groups, cut), g in zip(STRIDED, record([dict(fmha=s[0]) for s in STRIDED])):
+        first = g["launches"][0]
+        assert g["rc"] == 0 and first["kernel"] == kernel and len(g["launches"]) == 1 + cut, case
+        assert groups is None or first["args"][2] == groups, case
+        met.add((kernel, case[5], groups, cut))
+    assert len(met) == 8
+
+
 @pytest.mark.parametrize("causal", [0, 1])
 def test_workspace_holds_whole_ranges_and_is_bounded(causal):
     """splits x rows x (D + 2) floats, 2..64 splits, and splits x tiles within one round of the

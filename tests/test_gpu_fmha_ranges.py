@@ -72,6 +72,103 @@ def test_with_and_without_workspace(gpu, case):
     _check(host(o), host(l), ref, lref)
 
 
+STRIDED = [  # case, the kernel and its key groups, whether keys are cut (given a workspace)
+    ((2, 1, 4099, 16, 8, 256, True), "k_fmha_rows", None, True),
+    ((3, 2, 200, 8, 2, 128, True), "k_fmha_rows", None, False),
+    ((2, 31, 4000, 1, 1, 128, False), "k_fmha_rows", None, True),
+    ((1, 600, 600, 8, 2, 128, True), "k_fmha_fwd", 2, False),   # first tile: one key block
+    ((1, 130, 1500, 6, 2, 128, True), "k_fmha_fwd", 2, True),
+    ((2, 33, 2000, 4, 4, 256, True), "k_fmha_fwd", 1, True),
+    ((3, 300, 300, 4, 1, 256, True), "k_fmha_fwd", 1, False),
+    ((70, 40, 77, 8, 8, 128, True), "k_fmha_fwd", 1, False),
+]
+
+
+def _layout(x, how, gpu, fill):
+    """x [B, S, H, D] on the GPU in a wider buffer whose other elements hold `fill`."""
+    import torch
+
+    B, S, H, D = x.shape
+    if how == "bhsd":
+        buf = torch.full((B, H + 1, S + 5, D), fill, dtype=torch.float16, device=gpu)
+        v = buf[:, :H, :S].permute(0, 2, 1, 3)
+    else:  # a cache longer than S whose positions also hold other heads
+        buf = torch.full((B, S + 37, H + 3, D + 16), fill, dtype=torch.float16, device=gpu)
+        v = buf[:, :S, 1:H + 1, 8:8 + D]
+    v.copy_(dev(x, gpu))
+    return v, buf
+
+
+@pytest.mark.parametrize("how", ["bhsd", "cache"])
+@pytest.mark.parametrize("case", [s[0] for s in STRIDED],
+                         ids=lambda c: "b%d_q%d_k%d_h%d_kv%d_d%d_%d" % c)
+def test_strides_of_every_form(gpu, case, how):
+    """Every operand a view into a wider buffer.  NaN around Q, K and V (the cache past Sk too) must
+    not reach the result, and nothing around O may be written."""
+    import torch
+    from cuda_tempiler_amd import capi
+
+    B, Sq, Sk, H, Hkv, D, causal = case
+    Q, K, V = _inputs(B, Sq, Sk, H, Hkv, D, seed=17 * Sq + Sk)
+    scale = 1.0 / np.sqrt(D)
+    ref, lref = O.fmha_fwd(Q, K, V, scale, causal)
+    nan = float("nan")
+    (dQ, _), (dK, _), (dV, _) = (_layout(x, how, gpu, nan) for x in (Q, K, V))
+    dO, buf = _layout(Q, how, gpu, 7.0)
+    say("strided", how, case)
+    for ws in (True, False):
+        buf.fill_(7.0)
+        l = torch.empty((B, H, Sq), dtype=torch.float32, device=gpu)
+        if ws:
+            capi.fmha_fwd(dQ, dK, dV, scale, causal, O=dO, LSE=l)
+        else:
+            p = capi.fmha_params(dQ, dK, dV, dO, l, scale, causal)
+            capi._check(capi.lib().tempo_fmha_fwd_launch(p, capi._stream(None)), "launch")
+        torch.cuda.synchronize()
+        _check(host(dO.contiguous()), host(l), ref, lref)
+        dO.fill_(7.0)
+        assert torch.all(buf == 7.0)
+
+
+@pytest.mark.parametrize("case", [s[0] for s in STRIDED if s[0][1] > 1],
+                         ids=lambda c: "b%d_q%d_k%d_h%d_kv%d_d%d_%d" % c)
+def test_special_values_stay_in_their_head(gpu, case):
+    """An infinite key in KV head 0 of the first sequence, a NaN query row in its last head: the rows
+    that score the key are NaN, as is the query's row.  Rows of another (batch, KV head) have the bits
+    they have without them; rows that share a tile with them round against another reference."""
+    import torch
+    from cuda_tempiler_amd import capi
+
+    B, Sq, Sk, H, Hkv, D, causal = case
+    Q, K, V = (dev(x, gpu) for x in _inputs(B, Sq, Sk, H, Hkv, D, seed=3 * Sq + Sk))
+    want, lwant = capi.fmha_fwd(Q, K, V, 0.1, causal)
+    Q, K = Q.clone(), K.clone()
+    G = H // Hkv
+    j = Sk - 1 if not causal else Sk - Sq  # a key that every row sees
+    j = max(j, 0)
+    K[0, j, 0, 5] = float("inf")
+    Q[B - 1, Sq // 2, H - 1, 2] = float("nan")
+    got, lgot = capi.fmha_fwd(Q, K, V, 0.1, causal)
+    torch.cuda.synchronize()
+    say("special values", case)
+    hit = torch.zeros((B, Sq, H), dtype=torch.bool, device=gpu)
+    up = Q[0, :, :G, 5] > 0  # a score of +inf: the row's softmax is NaN (-inf: weight 0)
+    hit[0, :, :G] = up
+    hit[B - 1, Sq // 2, H - 1] = True
+    assert torch.isnan(got[hit]).all()
+    clean = torch.ones_like(hit)
+    clean[0, :, :G] = False
+    clean[B - 1, :, H - G:] = False
+    assert torch.equal(got[clean], want[clean])
+    if B > 1 or Hkv > 1:  # the query row's neighbours
+        near = ~hit[B - 1, :, H - G:]
+        a, b = got[B - 1, :, H - G:][near].double(), want[B - 1, :, H - G:][near].double()
+        assert float((a - b).norm()) <= TOL * float(b.norm())
+    c = clean.permute(0, 2, 1)
+    assert torch.equal(lgot[c], lwant[c])
+    assert torch.isfinite(got[0, :, :G][~up & ~hit[0, :, :G]]).all()
+
+
 def test_captured_decode_step(gpu):
     """A decode step whose keys are cut, recorded in a graph: the workspace belongs to the graph's
     pool, and every replay, between eager calls on other data, equals the eager result."""
