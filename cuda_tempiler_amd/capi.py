@@ -115,10 +115,14 @@ def _check(rc: int, what: str) -> None:
 
 
 def _stream(stream):
-    if stream is None:  # the raw handle: building a torch Stream object costs about 1 us
+    if stream is None:
         import torch
 
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        # the raw handle where torch has this (private) call: a Stream object costs about 1 us
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:
+            return raw(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
     if isinstance(stream, int):
         return _p(stream)
     return _p(stream.cuda_stream)

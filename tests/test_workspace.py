@@ -62,3 +62,17 @@ def test_workspace_argument_is_checked(capi):
     B = torch.zeros(64, 256, dtype=torch.float16)
     with pytest.raises(ValueError):
         capi.gemm_fp16(A, B, workspace="pool")  # only None, "torch" or a tensor
+
+
+def test_current_stream_without_torchs_private_call(capi, monkeypatch):
+    """The raw handle comes from a private name of torch; without it, from the Stream object."""
+    import types
+
+    import torch
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=0x77))
+    assert capi._stream(None).value == 0x77
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda dev: 0x99 + dev, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 2)
+    assert capi._stream(None) == 0x9b
