@@ -56,16 +56,8 @@ def instantiation(kind, p, epi=0):
         return "launch_stream<%d,%d,%d,%d%s>" % (p["MB"], p["R"], p["U"], p.get("A", 0), tail)
     if epi and kind == "ilv" and p.get("PLAN"):  # tile and split count by plan_tiles
         return "launch_ilv_plan_gu<%d,%d,%d>" % (p["GROUP"], p["XCD"], p["RSP"])
-    if epi and kind == "ilv" and p.get("TAIL"):  # output columns in two parts
-        return "launch_ilv_gu_tail<%d,%d,%d,%d,%d,%d,%d,%d,%d,%s>" % (
-            p["BM"], p["BN"], p["BK"], p["WM"], p["WN"], p["STAGES"], p["GROUP"], p["XCD"],
-            p["RSP"], ",".join(str(v) for v in _select().ILV_TAIL[p["TAIL"]]))
-    if epi and kind == "ilv":
-        return "launch_ilv_gu<%d,%d,%d,%d,%d,%d,%d,%d,%d>" % (
-            p["BM"], p["BN"], p["BK"], p["WM"], p["WN"], p["STAGES"], p["GROUP"], p["XCD"],
-            p["RSP"])
     if epi:
-        raise ValueError("the fused gate/up epilogue exists for the stream and interleaved kernels")
+        raise ValueError("the fused gate/up epilogue exists for the stream kernels and for plans")
     if kind == "ilv" and p.get("PLAN") and not p.get("SW"):
         return "launch_ilv_plan<%d,%d,%d>" % (p["GROUP"], p["XCD"], p["RSP"])
     if kind == "ilv" and p.get("PLAN"):  # a split-K row of its own: RATE in 1/100

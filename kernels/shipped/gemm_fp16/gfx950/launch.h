@@ -267,10 +267,8 @@ inline hipError_t launch_dma(const GemmParams& p, hipStream_t s) {
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP,
           int SW, int MINKT>
 hipError_t launch_ilv(const GemmParams& p, hipStream_t s, const Workspace& w);
-// The same kernel with the fused gate/up epilogue (p.N the output width, B 2N rows).
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP>
-hipError_t launch_ilv_gu(const GemmParams& p, hipStream_t s, const Workspace& w);
-// That row with the output columns in two parts (whole rounds, then TBM x TBN/2-column tiles).
+// The same kernel with the fused gate/up epilogue (p.N the output width, B 2N rows) and the output
+// columns in two parts (whole rounds, then TBM x TBN/2-column tiles).
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP,
           int TBM, int TBN, int TBK, int TWM, int TWN, int TSTAGES>
 hipError_t launch_ilv_gu_tail(const GemmParams& p, hipStream_t s, const Workspace& w);

@@ -53,15 +53,6 @@ hipError_t launch_ilv_gu_part(const GemmParams& p, hipStream_t s, int up) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP>
-hipError_t launch_ilv_gu(const GemmParams& p, hipStream_t s, const Workspace& w) {
-  if (w.need) {
-    *w.need = 0;
-    return hipSuccess;
-  }
-  return launch_ilv_gu_part<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP>(p, s, p.N);
-}
-
 // The fused gate/up row with the output columns in two parts: where the last round of tiles
 // (BN/2 output columns each) is at most a quarter full, the whole rounds run on the leading
 // columns and the remaining columns on TBM x TBN/2-column tiles -- four or more times as many --

@@ -82,16 +82,8 @@ def instantiation(kind, p, epi=0):
     if kind == "ilv8" and p.get("PLAN"):  # tile and split count by plan_tiles
         return "launch_ilv8_plan%s<%d,%d,%d>" % ("_gu" if epi else "", p["GROUP"], p["XCD"],
                                                  p["RSP"])
-    if epi and kind == "ilv8" and p.get("TAIL"):  # output columns in two parts
-        return "launch_ilv8_gu_tail<%d,%d,%d,%d,%d,%d,%d,%d,%d,%s>" % (
-            p["BM"], p["BN"], p["BK"], p["WM"], p["WN"], p["STAGES"], p["GROUP"], p["XCD"],
-            p["RSP"], ",".join(str(v) for v in _select().ILV8_TAIL[p["TAIL"]]))
-    if epi and kind == "ilv8":
-        return "launch_ilv8_gu<%d,%d,%d,%d,%d,%d,%d,%d,%d>" % (
-            p["BM"], p["BN"], p["BK"], p["WM"], p["WN"], p["STAGES"], p["GROUP"], p["XCD"],
-            p["RSP"])
     if epi:
-        raise ValueError("the fused gate/up epilogue exists for the stream and interleaved kernels")
+        raise ValueError("the fused gate/up epilogue exists for the stream kernels and for plans")
     if kind == "ilv8" and p.get("TAIL"):  # N in two parts: whole rounds, then the tail part
         return "launch_ilv8_tail<%d,%d,%d,%d,%d,%d,%d,%d,%d,%s>" % (
             p["BM"], p["BN"], p["BK"], p["WM"], p["WN"], p["STAGES"], p["GROUP"], p["XCD"],

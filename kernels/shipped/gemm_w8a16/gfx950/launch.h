@@ -511,10 +511,8 @@ inline bool ilv8_fill_fits(const W8A16Params& p) {
   const int nm = (p.M + BM - 1) / BM;
   return nm * (p.N / BN) <= CUS && nm > (p.M + 255) / 256;
 }
-// The same kernel with the fused gate/up epilogue (p.N the output width, 2N weight rows), and
-// that row with the output columns in two parts.
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP>
-hipError_t launch_ilv8_gu(const W8A16Params& p, hipStream_t s, const Workspace& w);
+// The same kernel with the fused gate/up epilogue (p.N the output width, 2N weight rows) and the
+// output columns in two parts.
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP,
           int TBM, int TBN, int TBK, int TWM, int TWN, int TSTAGES, int TSW, int TMINKT>
 hipError_t launch_ilv8_gu_tail(const W8A16Params& p, hipStream_t s, const Workspace& w);

@@ -97,15 +97,6 @@ hipError_t launch_ilv8_gu_part(const W8A16Params& p, hipStream_t s, int up) {
   return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD, int RSP>
-hipError_t launch_ilv8_gu(const W8A16Params& p, hipStream_t s, const Workspace& w) {
-  if (w.need) {
-    *w.need = 0;
-    return hipSuccess;
-  }
-  return launch_ilv8_gu_part<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP>(p, s, p.N);
-}
-
 // The fused gate/up row with the output columns in two parts, as launch_ilv8_tail (unsplit
 // tail tiles): the whole rounds of BM x BN/2-column tiles, then the remaining columns on
 // TBM x TBN/2-column tiles; both parts read their up rows p.N rows past their gate rows.
