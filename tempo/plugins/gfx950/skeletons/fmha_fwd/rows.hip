@@ -6,8 +6,9 @@
 // is nothing to share between waves but the rows: each wave streams key blocks of its own (block
 // lo + wave, + 4, ...) and keeps its own running max, sum and O; the four are merged through LDS
 // at the end.  What bounds it is HBM: every key and value is read once, by one workgroup, and
-// the matrix work of a 32-key block (0.45 us at D = 256) is a tenth of the time a CU's share of
-// the HBM rate takes to bring it (32 KiB at 28 GB/s).  So the layout serves the stream only:
+// the matrix work of a wave's 32-key block (0.45 us at D = 256) is a tenth of the time the CU's
+// share of the HBM rate takes to bring its four waves' blocks (128 KiB at 28 GB/s).  So the layout
+// serves the stream only:
 //   * a wave's K and V blocks have one LDS slot each (128 KiB per workgroup at D = 256, 64 KiB
 //     and two workgroups per CU at D = 128).  K(next) is copied as soon as the scores have read
 //     K, V(next) as soon as P.V has read V, so at least half of the LDS is always in flight;
@@ -16,11 +17,12 @@
 //   * the key range is cut into `chunk` blocks per workgroup (grid = ranges x KV heads x
 //     batch), so that a batch of a few sequences fills the 256 CUs; each range's unnormalised O,
 //     reference and sum go to the workspace in fp32 and k_fmha_combine merges them.
-//   * the copies carry the nontemporal policy: K and V pass once, and streams of cached loads
-//     stop at 5.9 TB/s here (8 sequences, 4099 keys, D = 256: 54 us cached, 47 nontemporal).
-// Measured (us; before: a 128-row tile of k_fmha_fwd per query head): 8 sequences x 4099 keys, 16
-// heads, 8 KV heads, D = 256: 149 -> 47 (5.7 TB/s); 32 x 4096: 339 -> 153 (7.0 TB/s); 32 x 2048,
-// 32 heads, D = 128: 195 -> 44; 1 x 32768: 689 -> 30; 1 x 512: 14.8 -> 6.7.
+//   * the copies carry the nontemporal policy, for K and V pass once (us, cached -> nontemporal, 16
+//     heads, 8 KV heads, D = 256: 8 sequences x 4099 keys 53 -> 47.5, 32 x 4096 174 -> 153; 32
+//     heads, D = 128, 32 x 2048 54 -> 45).
+// Measured (us; before: a 128-row tile of k_fmha_fwd per query head), the same heads: 8 x 4099
+// 149 -> 47.5 (5.7 TB/s); 32 x 4096 345 -> 153 (7.0 TB/s); 1 x 32768 1084 -> 54; 1 x 512 21 -> 12;
+// 32 heads, D = 128, 32 x 2048 196 -> 45.
 namespace fmha {
 
 template <int D, bool CAUSAL>
