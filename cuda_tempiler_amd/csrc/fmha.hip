@@ -5,6 +5,8 @@
 #include <limits.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace tempo_fmha {
 #include "common/cdna4.h"
 #include "fmha_fwd/kernel.hip"
@@ -33,10 +35,12 @@ bool applicable(const TempoFmhaParams& p) {
 
 // How a call runs: on k_fmha_rows (all packed rows of a (batch, KV head) fit one 32-row tile) or
 // on k_fmha_fwd with `kg` key groups per workgroup; its key blocks in ranges of `chunk` (one
-// workgroup each; INT_MAX: not cut), merged by k_fmha_combine over `splits` ranges.
+// workgroup each; INT_MAX: not cut), merged by k_fmha_combine over `splits` ranges.  `hg`: head groups
+// of k_fmha_fwd, Hkv (packed) or H; `apart`: H is the better one where keys are not cut.
 struct Plan {
   bool rows;
-  int kg, chunk, splits;
+  int kg, chunk, splits, hg;
+  bool apart;
 };
 
 static int tile_rows(const Plan& pl) { return pl.rows ? 32 : fmha::BQ; }
@@ -52,34 +56,55 @@ static size_t ws_bytes(const TempoFmhaParams& p, const Plan& pl) {
 //   * Rows: a workgroup passes 4 blocks (128 keys) in 1.0 (D = 128) or 2.1 (D = 256), and a cut
 //     costs the second kernel (3) and its pass over the ranges (0.25 each).  256 workgroups
 //     stream at the HBM's rate, so a cut never asks for a second round: at 8 sequences x 8 KV
-//     heads x 4096 keys, D = 128, 4 ranges take 27.1, 1 range 49.1, 8 ranges 28.4.
+//     heads x 4096 keys, D = 128, 4 ranges take 27.1, 1 range 49.1, 8 ranges 28.4.  At D = 256 more
+//     than 16 rows over at most 4 blocks (one a wave) stay on tiles: 8 rows of 4 heads over 96
+//     keys 9.3 here, 8.3 there.
 //   * Tiles, D = 128: workgroups of two key groups where the grid leaves CUs with at most two
 //     workgroups and the longest tile has 16 key blocks or more -- 120 against 134 at 256 tiles of
 //     203 blocks, 84 against 98 at 512 causal tiles of up to 128 -- else one group, two
 //     workgroups per CU (291 against 330 at 2048 tiles of 64 blocks, 12 against 18 at 512 of 3).
 //   * Tiles, cut: while ranges x tiles fit one round of the CUs and the blocks saved (0.47 each,
 //     1.07 at D = 256) pay for the partial results: written, read and merged at 4.5 TB/s plus
-//     3.5 for the second kernel (512 rows over 8192 keys, 16 heads, D = 256: 92 against 272).
+//     3.5 (5 at D = 256) for the second kernel (512 rows over 8192 keys, 16 heads, D = 256: 96
+//     against 265; 2 x 158 rows over 235 keys, 2 heads, D = 256: 18.5 cut, 16.9 whole).
+//   * Tiles of one head each where a round of the CUs holds them, they have few key blocks and no
+//     cut pays: a tile's Q and O pass its CU at 40 GB/s (qo), so 128 packed rows cost 3.3 at D = 256
+//     and 38 rows 1.0 (4 x 38 rows x 104 keys, 8 heads, 2 KV heads: 14.3 packed, 10.6 apart).
 static Plan plan(const TempoFmhaParams& p) {
   constexpr int kCus = 256;
   const int G = p.H / p.Hkv;
   const long R = (long)p.Sq * G, bh = (long)p.B * p.Hkv;
-  Plan pl = {R <= 32, 1, INT_MAX, 1};
   const int L = p.causal ? fmha::fmha_tile_blocks<true>(0, (int)R, (int)R, G, p.Sq, p.Sk)
                          : fmha::fmha_tile_blocks<false>(0, (int)R, (int)R, G, p.Sq, p.Sk);
+  Plan pl = {R <= 32 && (p.D == 128 || R <= 16 || L > 4), 1, INT_MAX, 1, p.Hkv, false};
   const long tiles = bh * (pl.rows ? 1 : (R + fmha::BQ - 1) / fmha::BQ);
   if (!pl.rows && p.D == 128 && tiles <= 2 * kCus && L >= 16) pl.kg = 2;
-  if (2 * tiles > kCus) return pl;
+  const double blk = p.D == 128 ? 0.47 : 1.07;
+  // a tile of r rows' Q and O; the longest tile of one head, in the last rows or the 128 before them
+  auto qo = [&](long r) { return (double)(r < fmha::BQ ? r : fmha::BQ) * p.D * 1e-4; };
+  const int nq = (p.Sq + fmha::BQ - 1) / fmha::BQ, last = p.Sq - (nq - 1) * fmha::BQ;
+  double own = L * blk + qo(last);
+  if (nq > 1) own = std::max(own, (L - (p.causal ? (last + 31) / 32 : 0)) * blk + qo(fmha::BQ));
+  pl.apart = !pl.rows && pl.kg == 1 && G > 1 && L <= 16 && (long)p.B * p.H * nq <= kCus &&
+             own < L * blk + qo(R);
+  if (2 * tiles > kCus) {
+    if (pl.apart) pl.hg = p.H;
+    return pl;
+  }
   const double rows = (double)bh * R;
   auto cost = [&](int n) {
     const int c = (L + n - 1) / n;
     if (pl.rows)
       return (c + 3) / 4 * (p.D == 128 ? 1.0 : 2.1) + (n > 1 ? 3 + 0.25 * n : 0);
-    return c * (p.D == 128 ? 0.47 : 1.07) + (n > 1 ? 3.5 + n * rows * p.D * 8 / 4.5e6 : 0);
+    return c * blk + (n > 1 ? (p.D == 128 ? 3.5 : 5.0) + n * rows * p.D * 8 / 4.5e6 : 0);
   };
   int best = 1;
   for (int n = 2; n <= 64 && n * tiles <= kCus && 4 * n <= L; ++n)
     if (cost(n) < cost(best)) best = n;
+  if (pl.apart && own <= cost(best) + qo(R)) {
+    pl.hg = p.H;
+    return pl;
+  }
   if (best > 1) {
     pl.chunk = (L + best - 1) / best;
     pl.splits = (L + pl.chunk - 1) / pl.chunk;
@@ -90,6 +115,7 @@ static Plan plan(const TempoFmhaParams& p) {
 // The same call without a workspace.
 static Plan whole(const TempoFmhaParams& p) {
   Plan pl = plan(p);
+  if (pl.splits > 1 && pl.apart) pl.hg = p.H;
   pl.chunk = INT_MAX;
   pl.splits = 1;
   return pl;
@@ -97,24 +123,24 @@ static Plan whole(const TempoFmhaParams& p) {
 
 template <int D, bool CAUSAL>
 static hipError_t run(const TempoFmhaParams& p, const Plan& pl, float* ws, hipStream_t s) {
-  const int R = p.Sq * (p.H / p.Hkv), BQ = tile_rows(pl);
-  // one workgroup per (key range, tile of packed rows, KV head, batch); heaviest causal tile first
-  const dim3 grid((unsigned)((R + BQ - 1) / BQ) * p.Hkv * p.B * pl.splits), blk(pl.rows ? 256 : 256 * pl.kg);
+  const int hg = pl.rows ? p.Hkv : pl.hg, R = p.Sq * (p.H / hg), BQ = tile_rows(pl);
+  // one workgroup per (key range, tile of rows, head group, batch); heaviest causal tile first
+  const dim3 grid((unsigned)((R + BQ - 1) / BQ) * hg * p.B * pl.splits), blk(pl.rows ? 256 : 256 * pl.kg);
   const float scale_log2 = p.scale * 1.4426950408889634f;
   float* const ml = ws ? ws + (size_t)pl.splits * p.B * p.H * p.Sq * D : nullptr;
-  auto go = [&](auto kernel) {
+  auto go = [&](auto kernel, auto... last) {
     hipLaunchKernelGGL(kernel, grid, blk, 0, s, static_cast<const _Float16*>(p.Q),
                        static_cast<const _Float16*>(p.K), static_cast<const _Float16*>(p.V),
                        static_cast<_Float16*>(p.O), p.LSE, p.B, p.H, p.Hkv, p.Sq, p.Sk, scale_log2,
                        p.q_sb, p.q_ss, p.q_sh, p.k_sb, p.k_ss, p.k_sh, p.v_sb, p.v_ss, p.v_sh,
-                       p.o_sb, p.o_ss, p.o_sh, pl.chunk, ws, ml);
+                       p.o_sb, p.o_ss, p.o_sh, pl.chunk, ws, ml, last...);
   };
   if (pl.rows)
     go(fmha::k_fmha_rows<D, CAUSAL>);
   else if (D == 128 && pl.kg == 2)
-    go(fmha::k_fmha_fwd<D, CAUSAL, D == 128 ? 2 : 1>);
+    go(fmha::k_fmha_fwd<D, CAUSAL, D == 128 ? 2 : 1>, hg, p.H / hg, hg / p.Hkv);
   else
-    go(fmha::k_fmha_fwd<D, CAUSAL, 1>);
+    go(fmha::k_fmha_fwd<D, CAUSAL, 1>, hg, p.H / hg, hg / p.Hkv);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || pl.splits <= 1) return e;
   const long rows = (long)p.B * p.H * p.Sq;

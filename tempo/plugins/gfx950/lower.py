@@ -63,7 +63,7 @@ _ENTRY = {
 _ENTRY["fmha"] = ("fmha::k_fmha_fwd", ("D", "CAUSAL"),
                   "const _Float16*, const _Float16*, const _Float16*, _Float16*, float*, int, int, "
                   "int, int, int, float, long, long, long, long, long, long, long, long, long, long, "
-                  "long, long, int, float*, float*",
+                  "long, long, int, float*, float*, int, int, int",
                   ("common/cdna4.h", "fmha_fwd/kernel.hip"))
 _BOOL = {("fmha", "CAUSAL")}  # template parameters of type bool (written true / false)
 NAMESPACE = "tempo::gen"

@@ -11,7 +11,8 @@
 // head); each wave owns 32 rows; key/value blocks of BKV2 keys):
 //   * Rows are packed over the query heads of a KV head (fmha_tile_blocks below): the heads share
 //     the K and V blocks their tile brings in, a causal tile spans 128 / G positions instead of
-//     128, and few positions fill a tile with heads (C5, D = 256: 175 -> 168 us).
+//     128, and few positions fill a tile with heads (4096 keys, 16 heads, 8 KV heads, D = 256:
+//     165.5 -> 161 us).
 //   * S^T = K . Q^T on v_mfma_f32_32x32x16_f16: K rows are the "A" operand, Q rows the "B"
 //     operand, so every lane's result registers belong to ONE query row (column = lane % 32) --
 //     row max and row sum are in-lane plus one exchange with lane ^ 32.  Q stays in registers
@@ -68,7 +69,7 @@ __device__ __host__ __forceinline__ int fmha_tile_blocks(int r0, int rows, int R
   int kend = Sk;
   if (CAUSAL) {
     const int end = r0 + rows < R ? r0 + rows : R;
-    const int seen = (end - 1) / G + 1 + Sk - Sq;  // keys the tile's last row sees
+    const int seen = (G == 1 ? end - 1 : (end - 1) / G) + 1 + Sk - Sq;  // by the tile's last row
     kend = seen < Sk ? seen : Sk;
     if (kend < 0) kend = 0;
   }
@@ -117,13 +118,19 @@ __device__ __forceinline__ void fmha_buf_lds16(const void* base, unsigned nrec, 
 // instruction order hides a latency.  At D = 128 the kernel is held to 256 registers and two
 // waves share a SIMD, one issuing its softmax while the other's matrix instructions run: with one
 // wave the issue of MFMA, VALU, LDS and scalar instructions adds up (B = 1, 32 heads, 8 KV heads,
-// 8192 keys, causal: 741 us with one wave, 555 us with two, 0.99 PFLOP/s).  The two waves come
+// 8192 keys, causal: 748 us with one wave, 568 us with two, 0.97 PFLOP/s).  The two waves come
 // from two workgroups per CU or (KG = 2) from one of eight waves whose two groups of four take half
 // of the key blocks each, with K and V slots of their own, and merge through LDS: the form for
 // grids that put at most two workgroups on a CU, where it needs no second pass over partial
-// results (B = 2, 500 rows, 6500 keys: 147 us before, 134 with two workgroups per CU, 120 with two
+// results (B = 2, 500 rows, 6500 keys: 146 us before, 134 with two workgroups per CU, 119 with two
 // groups).  256-row tiles on eight waves and 64 rows per wave were within 3 % of the two-workgroup
 // form, and reading the next block's first fragments at the end of the chain within 1 %.
+//
+// `Hg` head groups of G = H / Hg query heads, gk = Hg / Hkv groups a KV head: Hg = Hkv packs the query
+// heads of a KV head as above; Hg = H gives every head tiles of its own, for grids that leave CUs idle and have few key blocks.  There a workgroup's time is its CU's
+// intake of Q and store of O (64 KiB each for 128 rows at D = 256), which packing only concentrates
+// (us, packed -> one head a tile, D = 256: 4 sequences x 64 rows and keys, 16 heads, 8 KV heads
+// 12.3 -> 9.9; 1 x 16 rows x 203 keys, 64 heads 16.9 -> 13.1).
 //
 // `chunk` < the tile's key blocks: the grid holds one workgroup per (tile, range of chunk blocks),
 // each writing its unnormalised O, reference and sum to the workspace for k_fmha_combine
@@ -169,7 +176,7 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
     const _Float16* __restrict__ Vg, _Float16* __restrict__ O, float* __restrict__ LSE, int B,
     int H, int Hkv, int Sq, int Sk, float scale_log2, long q_sb, long q_ss, long q_sh, long k_sb,
     long k_ss, long k_sh, long v_sb, long v_ss, long v_sh, long o_sb, long o_ss, long o_sh,
-    int chunk, float* __restrict__ part, float* __restrict__ part_ml) {
+    int chunk, float* __restrict__ part, float* __restrict__ part_ml, int Hg, int G, int gk) {
   static_assert(D == 128 || D == 256, "head dim 128 or 256");
   constexpr int BKV2 = 32;
   constexpr int WAVES = 4;     // per key group
@@ -205,13 +212,15 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
   const int hl = lane >> 5;
   const int l32 = lane & 31;
 
-  const int G = H / Hkv, R = Sq * G;
+  // (a division costs a lone workgroup 0.1 us, so the host does what it can)
+  const int R = Sq * G;
   const int nqb = (R + BQW - 1) / BQW;
-  const int per = Hkv * B * nqb;
-  const int sp = blockIdx.x / per, bid = blockIdx.x % per;
-  const int qb = CAUSAL ? (nqb - 1 - bid / (Hkv * B)) : bid / (Hkv * B);
-  const int hb = bid % (Hkv * B);
-  const int hk = hb % Hkv, b = hb / Hkv;
+  const int per = Hg * B * nqb;
+  const int sp = (int)blockIdx.x < per ? 0 : blockIdx.x / per, bid = blockIdx.x - sp * per;
+  const int tile = bid / (Hg * B), hb = bid - tile * (Hg * B);
+  const int qb = CAUSAL ? nqb - 1 - tile : tile;
+  const int b = hb / Hg, hg = hb - b * Hg;
+  const int hk = gk == 1 ? hg : hg / gk;
   const int r0 = qb * BQW;
   // the tile's key blocks, this workgroup's [lo, lo + nwg), and this key group's: the groups take
   // ceil(nwg / KG) blocks each; where the last has fewer, its blocks past the range re-read the
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
   const int nkb = (nwg + KG - 1) / KG;
   const int lo = wlo + kg * nkb;
   const int jlast = wlo + nwg - 1 - lo;  // last block of the range, from this group's first
-  const int q0 = r0 / G;
+  const int q0 = G == 1 ? r0 : r0 / G;
   Sk -= lo * BKV2;  // keys counted from this group's first block
   const int off = Sk - Sq;
   const int kstop = KG > 1 ? min(Sk, (jlast + 1) * BKV2) : Sk;  // first key that is not its own
@@ -232,8 +241,8 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
   const char* Vp = reinterpret_cast<const char*>(Vg + b * v_sb + (long)hk * v_sh + (long)lo * BKV2 * v_ss);
 
   const int row = min(r0 + wave * 32 + l32, R - 1);
-  const int qi = row / G;
-  const _Float16* Qp = Q + b * q_sb + (long)(hk * G + row % G) * q_sh + (long)qi * q_ss;
+  const int qi = G == 1 ? row : row / G, g = row - qi * G;  // position, head of the group
+  const _Float16* Qp = Q + b * q_sb + (long)(hg * G + g) * q_sh + (long)qi * q_ss;
   f16x8 qf[DS];
 #pragma unroll
   for (int st = 0; st < DS; ++st) qf[st] = *reinterpret_cast<const f16x8*>(Qp + 16 * st + 8 * hl);
@@ -513,7 +522,7 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
   if (nkt > chunk) {
     // other workgroups hold key blocks of this tile too: unnormalised O, its reference and its
     // sum; k_fmha_combine merges them
-    const long pr = (long)sp * B * Hkv * R + (long)hb * R + row;
+    const long pr = (long)sp * B * Hg * R + (long)hb * R + row;
     float* po = part + pr * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -528,7 +537,7 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
     return;
   }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  const int h = hk * G + row % G;
+  const int h = hg * G + g;
   _Float16* Op = O + b * o_sb + (long)qi * o_ss + (long)h * o_sh;
 #pragma unroll
   for (int db = 0; db < DB; ++db)

@@ -36,6 +36,26 @@ def test_strided_gpu_cases_reach_every_form():
     assert len(met) == 8
 
 
+@pytest.mark.parametrize("case,tiles", [
+    ((4, 38, 104, 8, 2, 256, True), 4 * 8),        # a head's rows a tile
+    ((2, 127, 129, 6, 2, 128, False), 2 * 6),
+    ((8, 32, 250, 32, 2, 256, True), 8 * 32),      # ... B x H at the CUs' count
+    ((9, 40, 60, 32, 2, 256, True), 9 * 2 * 5),    # past it: 16 heads' rows packed, 5 tiles of 128
+    ((4, 128, 104, 8, 2, 256, True), 4 * 2 * 4),   # whole tiles either way: packed
+    ((1, 187, 187, 8, 4, 256, True), 8 * 2),       # a short last tile, the longest one
+    ((1, 187, 187, 8, 4, 256, False), 4 * 3),      # every tile as long: packed
+    ((1, 8, 96, 4, 1, 256, True), 4),              # few rows, few blocks: not the few-rows kernel
+    ((1, 8, 160, 4, 1, 256, True), 1),             # its five blocks: that kernel
+    ((4, 38, 104, 8, 8, 256, True), 4 * 8),        # nothing to pack
+])
+def test_which_tiles_pack_heads(case, tiles):
+    """Without a workspace: one workgroup per (batch, head group, tile)."""
+    from tests.launch_recorder import record
+
+    g = record([dict(fmha=case, entry="none")])[0]
+    assert [l["grid"] for l in g["launches"]] == [tiles] and g["rc"] == 0
+
+
 @pytest.mark.parametrize("causal", [0, 1])
 def test_workspace_holds_whole_ranges_and_is_bounded(causal):
     """splits x rows x (D + 2) floats, 2..64 splits, and splits x tiles within one round of the

@@ -31,6 +31,10 @@ CASES = [
     (1, 300, 513, 4, 2, 128, False),
     (1, 1000, 520, 2, 1, 128, True),    # tiles without keys beside tiles of two key groups
     (70, 40, 77, 8, 8, 128, True),      # one key group: short tiles, more than two per CU
+    (4, 38, 104, 8, 2, 256, True),      # a head's rows a tile: few blocks on an idle part
+    (1, 16, 203, 32, 4, 256, True),
+    (2, 127, 129, 6, 2, 128, False),
+    (8, 120, 250, 32, 2, 256, True),    # (B x H at the CUs' count)
 ]
 
 
@@ -81,6 +85,8 @@ STRIDED = [  # case, the kernel and its key groups, whether keys are cut (given 
     ((2, 33, 2000, 4, 4, 256, True), "k_fmha_fwd", 1, True),
     ((3, 300, 300, 4, 1, 256, True), "k_fmha_fwd", 1, False),
     ((70, 40, 77, 8, 8, 128, True), "k_fmha_fwd", 1, False),
+    ((4, 38, 104, 8, 2, 256, True), "k_fmha_fwd", 1, False),    # a head's rows a tile
+    ((2, 127, 129, 6, 2, 128, False), "k_fmha_fwd", 1, False),
 ]
 
 
