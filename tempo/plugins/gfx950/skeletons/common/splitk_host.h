@@ -217,6 +217,7 @@ inline hipError_t launch_reduce(const float* ws, int splits, int M, int N, _Floa
     case 5: run_reduce<5>(ws, splits, M, N, C, ldc, s); break;
     case 6: run_reduce<6>(ws, splits, M, N, C, ldc, s); break;
     case 7: run_reduce<7>(ws, splits, M, N, C, ldc, s); break;
+    case 1: run_reduce<1>(ws, splits, M, N, C, ldc, s); break;
     default: run_reduce<8>(ws, splits, M, N, C, ldc, s);
   }
   return hipGetLastError();

@@ -269,3 +269,24 @@ def test_gate_up_plan_against_oracle(gpu, fmt, case):
         r = O.rel_l2(host(C), ref)
         say("fmt", fmt, "case", case, "need", _gate_up_need(fmt, M, N, K), what, "relL2 %.3e" % r)
         assert r <= 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [2, 3, 7, 8, 9, 10, 11, 12, 13, 15, 16, 17, 27, 31])
+def test_reduction_of_every_remainder(gpu, splits):
+    """The reduction takes the splits in eights and then the rest: one 128-column tile of the 64-row
+    split-K row, whose split count is K / 512."""
+    import torch
+    from tests.gpu_util import host, say
+
+    M, N, K = 40, 128, 512 * splits
+    assert capi.route(0, M, N, K) == "i64x128k64s4w256"
+    assert capi.workspace_bytes(0, M, N, K) == splits * M * N * 4
+    A = O.randn_f16((M, K), 3 + splits, K ** -0.5)
+    B = O.randn_f16((N, K), 5, 1.0)
+    dA, dB = _dev(gpu, A, B)
+    C = capi.gemm_fp16(dA, dB)
+    torch.cuda.synchronize()
+    r = O.rel_l2(host(C), O.gemm_f16(A, B))
+    say("splits", splits, "relL2 %.3e" % r)
+    assert r <= 5e-4
