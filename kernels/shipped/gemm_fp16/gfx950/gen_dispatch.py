@@ -155,7 +155,7 @@ def render_prefill() -> str:
                    % inst)
     if any(r[4].get("PLAN") for r in sel.LADDER):
         out.append("template bool plan_instead<8,1,8>(const GemmParams&, hipStream_t, const Workspace&, "
-                   "double, double, size_t, hipError_t*);")
+                   "const OwnRow&, hipError_t*);")
     return "\n".join(out) + "\n"
 
 

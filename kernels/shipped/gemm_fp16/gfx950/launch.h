@@ -295,12 +295,20 @@ inline constexpr PlanTable kPlanTables[] = {
 #include "plan.inc"
 };
 #undef TEMPO_TABLE
-// The plan in place of a row whose own time is estimated at own_us and which needs own_bytes of
-// workspace: true (with *e) where the plan is below `ahead` of it, the interleaved kernel takes the
-// shape and the plan's workspace can be had (workspace_to_gain).
+// A row's own side of the choice between it and the plan: its estimated microseconds and workspace,
+// the part of `us` that the plan (split: `ahead_split`) has to stay below, and what the plan's
+// estimate is corrected by, us a workgroup and us a million weights at least.
+struct OwnRow {
+  double us;
+  size_t bytes;
+  double ahead, ahead_split;
+  double wg = 0, weights = 0;
+};
+// The plan in place of a row: true (with *e) where it is that far ahead, the interleaved kernel takes
+// the shape and the plan's workspace can be had (workspace_to_gain).
 template <int GROUP, int XCD, int RSP>
-bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double own_us,
-                  double ahead, size_t own_bytes, hipError_t* e);
+bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, const OwnRow& own,
+                  hipError_t* e);
 
 // One dispatch row: launchers without a workspace ignore it (and, asked for their need, report 0).
 inline hipError_t call_row(hipError_t (*f)(const GemmParams&, hipStream_t), const GemmParams& p,
@@ -316,13 +324,18 @@ inline hipError_t call_row(hipError_t (*f)(const GemmParams&, hipStream_t, const
   return f(p, s, w);
 }
 
-// An unsplit row, or the plan where that is ahead.
+// An unsplit row, or the plan where that is ahead.  At M <= 128 and weight rows a multiple of 16 KiB
+// apart, where a tile's rows fall on few HBM channels, it has to be 30 % ahead ((65, 15360, 8192) 58 us
+// on the row, 74 planned; (65, 17408, 8192) 103 against 69).  At M > 128 a split plan has to be further ahead:
+// the table takes its partial sums and weights for about 15 % too little when the weights come from
+// HBM ((256, 15360, 11008) 118 us on the row, 133 in two splits; (129, 13824, 8192) 78 against 72).
 template <int BM, int BN, int BK, int WM, int WN, int STAGES, int SWZ, int GROUP, int XCD, int MS,
           int RATE100>
 inline hipError_t launch_dma_or_plan(const GemmParams& p, hipStream_t s, const Workspace& w) {
   hipError_t e = hipSuccess;
   const double own = tile_us(plan_table(kPlanTables, p.M), RATE100 * 0.01, BM, BN, BK, p.M, p.N, p.K, 1);
-  if (plan_instead<8, 1, 8>(p, s, w, own, p.M <= 128 ? 0.85 : 0.95, 0, &e)) return e;
+  const double ahead = p.M > 128 ? 0.95 : p.ldb % 8192 == 0 ? 0.7 : 0.85;
+  if (plan_instead<8, 1, 8>(p, s, w, {own, 0, ahead, p.M <= 128 ? ahead : 0.8}, &e)) return e;
   if (w.need) {
     *w.need = 0;
     return hipSuccess;
@@ -330,19 +343,28 @@ inline hipError_t launch_dma_or_plan(const GemmParams& p, hipStream_t s, const W
   return launch_dma<BM, BN, BK, WM, WN, STAGES, SWZ, GROUP, XCD, MS>(p, s);
 }
 
-// Estimated microseconds of a line row: every group of 16 SN weight rows takes in its weights and
-// the activations (at M <= 16 half of the padding too), at 9.7 (M <= 16) or 10.5 TB/s over the part
-// in whole rounds of groups over the CUs; a k-slice row's second kernel 5.  Within 15 % of M = 4 ..
-// 32, N = 2560 .. 11008, K = 2560 .. 17408; too low past M = 32, where the plan wins by far more.
+// Estimated microseconds of a line row.  M <= 16: a fit to 259 shapes (M = 2 .. 16, N = 512 ..
+// 11264, K = 512 .. 18944, weights from HBM), -12 to +11 % at the 5th and 95th percentile: one round of
+// workgroups takes in 16 weight rows and the activations each, several share the HBM's rate.  Above:
+// every group of 16 SN weight rows takes in its weights and the activations at 10.5 TB/s over the part
+// in whole rounds of groups over the CUs; a k-slice row's second kernel 5.  Too low past M = 32, where
+// the plan wins by far more.
 inline double line_us(const GemmParams& p, int mb, int sn, int ks) {
   const int wgs = p.N / (16 * sn);
   const long w = (long)wgs * ks;
-  const int rows = 16 * sn + (mb == 1 ? (16 + p.M) / 2 : p.M);
-  const double mbytes = (double)wgs * p.K * 2e-6 * rows;
-  return 3 + (mb == 1 ? 0.103 : 0.095) * mbytes * (double)((w + 255) / 256 * 256) / (double)w + (ks > 1 ? 5 : 0);
+  const long rounds = (w + 255) / 256;
+  if (mb == 1 && rounds == 1) return 2.5 + 1.5 * w / 256 + (0.89 + 0.037 * p.M) * p.K * 1e-3;
+  if (mb == 1) return 5.8 + rounds * (1.1 + 0.029 * p.M) * p.K * 1e-3;
+  const double mbytes = (double)wgs * p.K * 2e-6 * (16 * sn + p.M);
+  return 3 + 0.095 * mbytes * (double)(rounds * 256) / (double)w + (ks > 1 ? 5 : 0);
 }
 
-// A line row (KS > 1: with k slices), or the plan where that is ahead.
+// A line row (KS > 1: with k slices), or the plan where that is ahead.  At M <= 16 the two are close,
+// and the table is low for few rows: a plan's workgroups start over about 2.5 us (0.01 each) and its
+// split weight rows come from HBM at 4.35 TB/s at most (0.46 a million).  Corrected so, and 7 % ahead,
+// none of 96 planned shapes was slower than its row, and five that would gain 8 to 17 % stay on it;
+// uncorrected, 28 were slower, up to 1.27 times ((2, 3072, 6144) 9.9 us on the row, 12.5 planned;
+// (4, 11008, 11008) 45 against 54).
 template <int MB, int R, int D, int SN, int WAVES, int KS>
 inline hipError_t launch_line_or_plan(const GemmParams& p, hipStream_t s, const Workspace& w) {
   hipError_t e = hipSuccess;
@@ -351,7 +373,9 @@ inline hipError_t launch_line_or_plan(const GemmParams& p, hipStream_t s, const 
   const bool aliased = p.M <= 32 && p.ldb % 8192 == 0;
   const int ks = KS > 1 ? line_kslices(p.N / (16 * R * SN), p.K, KS) : 1;
   const size_t own = ks > 1 ? (size_t)ks * p.M * p.N * sizeof(float) : 0;
-  if (!aliased && plan_instead<8, 1, 8>(p, s, w, line_us(p, MB, SN, ks), 0.88, own, &e)) return e;
+  const double us = line_us(p, MB, SN, ks);
+  const OwnRow row = MB == 1 ? OwnRow{us, own, 0.93, 0.93, 0.01, 0.46} : OwnRow{us, own, 0.88, 0.88};
+  if (!aliased && plan_instead<8, 1, 8>(p, s, w, row, &e)) return e;
   if constexpr (KS > 1) {
     return launch_line_ks<MB, R, D, SN, WAVES, KS>(p, s, w);
   } else {

@@ -114,10 +114,42 @@ hipError_t run_plan(const GemmParams& p, hipStream_t s, float* ws, const TilePla
   return hipErrorInvalidConfiguration;
 }
 
+// plan_tiles over `cols` weight rows, but for 192 x 256 tiles (5) whose tile rows make whole raster
+// groups of 8 and a ragged one: those run at 0.82 to 1.05 PFLOP/s, whatever their round's fill, where
+// 256 x 256 tiles (2) in whole groups reach 1.1.  So from K = 3584 on the 256-row tiles take what the
+// 192-row ones would need longer for at 1 PFLOP/s, and what leaves their own last round of whole
+// groups at most 32 tiles (us, 256 rows against 192: (2048, 11008, 11008) 478, 539; (2048, 11264,
+// 13824) 582, 660; (2048, 9216, 12288) 491, 516; (2048, 17408, 11008) 724, 871; where they stay:
+// (2048, 10240, 3584) 162, 141; in whole groups: (3000, 11008, 11008) 819, 628).
+// Fused gate/up (cols = 2N): at M <= 128 a split has to be 10 % ahead of the best unsplit tile, whose
+// short last round costs less than a whole one ((74, 17408, 3840) 66 us unsplit, 71 in three splits);
+// and where the gate and the up panel lie an odd number of 128 rows of a multiple of 8 KiB apart, the
+// 192-row tiles give way to 256 rows ((700, 14464, 4096) 189 against 230).
+inline TilePlan ilv_plan(const GemmParams& p, int cols, bool split) {
+  TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, split);
+  if (cols != p.N && p.M <= 128 && pl.splits > 1) {
+    const TilePlan flat = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, false);
+    if (flat.tile >= 0 && pl.us > 0.9 * flat.us) pl = flat;
+  }
+  if (cols != p.N && pl.tile == 5 && pl.splits == 1 && p.N % 256 && p.ldb % 4096 == 0) pl.tile = 2;
+  const int nm5 = (p.M + 191) / 192, nm = (p.M + 255) / 256;
+  if (pl.tile != 5 || pl.splits != 1 || p.K < 3584 || p.K % 64 || nm5 < 8 || nm5 % 8 == 0) return pl;
+  double rate = 0;
+  for (const TileRate& r : plan_table(kPlanTables, p.M).rate)
+    if (r.tile == 2) rate = r.us[0];
+  const double us = tile_us(plan_table(kPlanTables, p.M), rate, 256, 256, 64, p.M, cols, p.K, 1);
+  const int rest = (int)((long)nm * (cols / 256) % 256);
+  if (2e-9 * p.M * cols * p.K > us || (nm % 8 == 0 && rest > 0 && rest <= 32)) {
+    pl.tile = 2;
+    pl.us = us;
+  }
+  return pl;
+}
+
 template <int GROUP, int XCD, int RSP>
 hipError_t launch_ilv_planned(const GemmParams& p, hipStream_t s, const Workspace& w, bool gate_up) {
   const int cols = gate_up ? 2 * p.N : p.N;
-  TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, true);
+  TilePlan pl = ilv_plan(p, cols, true);
   const size_t bytes = pl.splits > 1 ? (size_t)pl.splits * p.M * cols * sizeof(float) : 0;
   if (w.need) {
     *w.need = bytes;
@@ -127,7 +159,7 @@ hipError_t launch_ilv_planned(const GemmParams& p, hipStream_t s, const Workspac
   if (bytes) {
     hipError_t err = hipSuccess;
     ws = workspace_to_gain(w, bytes, 0, s, &err);
-    if (!ws.ptr) pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, cols, p.K, false);  // unsplit
+    if (!ws.ptr) pl = ilv_plan(p, cols, false);  // unsplit
   }
   return run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, gate_up);
 }
@@ -138,12 +170,16 @@ hipError_t launch_ilv_plan(const GemmParams& p, hipStream_t s, const Workspace& 
 }
 
 template <int GROUP, int XCD, int RSP>
-bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double own_us,
-                  double ahead, size_t own_bytes, hipError_t* e) {
+bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, const OwnRow& own,
+                  hipError_t* e) {
   constexpr int kLd = 0x7fffffff / (2 * 256);
   if (p.lda > kLd || p.ldb > kLd) return false;
   const TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, p.N, p.K, true);
-  if (pl.tile < 0 || pl.us >= ahead * own_us) return false;
+  if (pl.tile < 0) return false;
+  const TileDims& d = kPlanTiles[pl.tile];
+  const double wgs = (double)((p.M + d.bm - 1) / d.bm) * (p.N / d.bn) * pl.splits;
+  const double us = std::max(pl.us + own.wg * wgs, own.weights * 1e-6 * p.N * p.K);
+  if (us >= (pl.splits > 1 ? own.ahead_split : own.ahead) * own.us) return false;
   const size_t bytes = pl.splits > 1 ? (size_t)pl.splits * p.M * p.N * sizeof(float) : 0;
   *e = hipSuccess;
   if (w.need) {
@@ -152,7 +188,7 @@ bool plan_instead(const GemmParams& p, hipStream_t s, const Workspace& w, double
   }
   Lease ws;
   if (bytes) {
-    ws = workspace_to_gain(w, bytes, own_bytes, s, e);
+    ws = workspace_to_gain(w, bytes, own.bytes, s, e);
     if (!ws.ptr) return false;
   }
   *e = run_plan<GROUP, XCD, RSP>(p, s, ws.ptr, pl, false);
@@ -164,12 +200,10 @@ template <int BM, int BN, int BK, int WM, int WN, int STAGES, int GROUP, int XCD
 hipError_t launch_ilv_or_plan(const GemmParams& p, hipStream_t s, const Workspace& w) {
   const int splits = split_count((p.M + BM - 1) / BM * (p.N / BN), p.K / BK, SW, MINKT);
   hipError_t e = hipSuccess;
-  if (plan_instead<GROUP, XCD, RSP>(p, s, w,
-                                    tile_us(plan_table(kPlanTables, p.M), RATE100 * 0.01, BM, BN, BK,
-                                            p.M, p.N, p.K, splits), 0.95,
-                                    splits > 1 ? (size_t)splits * p.M * p.N * sizeof(float) : 0,
-                                    &e))
-    return e;
+  const OwnRow own = {tile_us(plan_table(kPlanTables, p.M), RATE100 * 0.01, BM, BN, BK, p.M, p.N, p.K,
+                              splits),
+                      splits > 1 ? (size_t)splits * p.M * p.N * sizeof(float) : 0, 0.95, 0.95};
+  if (plan_instead<GROUP, XCD, RSP>(p, s, w, own, &e)) return e;
   return launch_ilv<BM, BN, BK, WM, WN, STAGES, GROUP, XCD, RSP, SW, MINKT>(p, s, w);
 }
 
@@ -180,7 +214,7 @@ hipError_t launch_ilv_plan_gu(const GemmParams& p, hipStream_t s, const Workspac
   const int nm = (p.M + 255) / 256, tiles = nm * (p.N / 128), whole = tiles / 256 * 256;
   if (p.M > 128 && p.N % 128 == 0 && whole > 0 && whole % nm == 0 && whole < tiles &&
       4 * (tiles - whole) <= 256) {
-    const TilePlan pl = plan_tiles(kPlanTiles, kPlanTables, 0, p.M, 2 * p.N, p.K, true);
+    const TilePlan pl = ilv_plan(p, 2 * p.N, true);
     double r256 = 0, r128 = 0;
     for (const TileRate& r : plan_table(kPlanTables, 1 << 30).rate) {
       if (r.tile == 2) r256 = r.us[0];

@@ -61,10 +61,10 @@ LADDER = [
     # (16, 3840, 15360); 0.99x at M = 8)
     (16, 0, "l1r1n4d4k8", "line", dict(MB=1, R=1, D=4, SN=4, W=2048, KS=8, KMIN=12288)),
     # PLAN on a line row: the interleaved kernel's 64-row tiles with split-K where they are estimated
-    # 12 % ahead of the row (line_us) and get their workspace.  The row's cost is the activations
-    # every 16 weight rows take in again: (8, 5120, 5120) 17.4 -> 13.3 us, (32, 5120, 5120) 25 -> 15,
-    # (32, 11008, 4096) 31 -> 23, (32, 5120, 17408) 42 -> 34, (64, 7168, 5120) 37 -> 21; at N = 15360
-    # and (16, 4096, 4096) the rows stay ahead
+    # ahead of the row (line_us; 7 % at M <= 16, 12 % above) and get their workspace.  The row's cost
+    # is the activations every 16 weight rows take in again: (8, 5120, 5120) 17.6 -> 13.9 us,
+    # (32, 5120, 5120) 25 -> 15, (32, 11008, 4096) 32 -> 23, (32, 5120, 17408) 43 -> 36,
+    # (64, 7168, 5120) 37 -> 21; at N = 15360 and (16, 4096, 4096) the rows stay ahead
     (16, 0, "l1r1d4", "line", dict(MB=1, R=1, D=4, W=2048, PLAN=1)),
     (16, 0, "s16r1u4", "stream", dict(MB=1, R=1, U=4, A=0)),
     # 16 < M <= 32, wide N: LDS-DMA tiles of 64 weight rows that take 256 k per stage (512
@@ -99,13 +99,15 @@ LADDER = [
     # 128-k stages (256 contiguous bytes of each weight row per copy): 1.01-1.06x the 64-k
     # four-stage row at M = 100, 128 (15360, 3840) and 128 (12288, 4096); at M = 200-256 the
     # 128 x 128 tiles of 128 k lose (0.92-0.97x), so the M <= 256 rows keep 64 k
+    # (RATE: 79 shapes of M = 65 .. 128 take 6.1 to 8.3; 6.8 keeps (80, 13824, 8192), 56 us here and 68
+    # planned, and (128, 15360, 8192), 62 and 68)
     (128, 12288, "d128x64k128s3", "dma",
      dict(BM=128, BN=64, BK=128, WM=2, WN=2, STAGES=3, SWZ=1, GROUP=8, XCD=1, MS=16, PLAN=1,
-          RATE=8.2)),
+          RATE=6.8)),
     (128, 12288, "d128x64k64s4", "dma",
      dict(BM=128, BN=64, BK=64, WM=2, WN=2, STAGES=4, SWZ=1, GROUP=8, XCD=1, MS=16)),
-    # (PLAN at 64 < M <= 128: (128, 34816, 5120) 116 -> 91 us on 128 x 256 tiles, (96, 11008, 4096)
-    # 34 -> 31, (128, 4096, 4096) 17.4 -> 15.0, (96, 2560, 2560) 13.2 -> 10.5)
+    # (PLAN at 64 < M <= 128: (128, 34816, 5120) 115 -> 91 us on 128 x 256 tiles, (96, 11008, 4096)
+    # 34 -> 31, (128, 4096, 4096) 17.7 -> 15.3, (96, 2560, 2560) 14.8 -> 12.3)
     (128, 0, "i128x128k64s3w256", "ilv",
      dict(BM=128, BN=128, BK=64, WM=2, WN=2, STAGES=3, GROUP=8, XCD=1, RSP=8, SW=256, MINKT=8,
           NMAX=6144, PLAN=1, RATE=10.6)),
@@ -114,10 +116,10 @@ LADDER = [
           RATE=4.5)),
     (128, 0, "l8r1n2d3", "line", dict(MB=8, R=1, D=3, SN=2, W=2048)),
     # PLAN rows: the launcher picks the tile and the split count by plan(); the row's own tile names
-    # it and, with RATE (its own us per 1000 k and round), runs unless the plan is 5 % ahead.  At
-    # 128 < M <= 256 the plan is up to 1.4x the single tiles ((160, 11008, 4096): 50 -> 37 us); at
-    # M > 256 it is 2.0x on average up to M = 1024 and 1.05x from there ((512, 5120, 17408): 331 ->
-    # 110 us, (1024, 1024, 5120): 88 -> 23)
+    # it and, with RATE (its own us per 1000 k and round), runs unless the plan is 5 % ahead (split:
+    # 20 % on the two LDS-DMA rows).  Random shapes with the weights from HBM, single tiles against the
+    # plan, geometric means: 1.29x at 128 < M <= 256 ((160, 11008, 4096): 50 -> 36 us), 1.88x up to
+    # M = 1024 and 1.26x from there ((512, 5120, 17408): 331 -> 117 us, (1024, 1024, 5120): 108 -> 24)
     (256, 12288, "d128x128k64s4", "dma",
      dict(BM=128, BN=128, BK=64, WM=2, WN=2, STAGES=4, SWZ=1, GROUP=8, XCD=1, MS=16, PLAN=1,
           RATE=10.2)),
@@ -154,13 +156,10 @@ LADDER_GATE_UP = [
     (128, 0, "gi128x256k64s3", "ilv",
      dict(BM=128, BN=256, BK=64, WM=1, WN=4, STAGES=3, GROUP=8, XCD=1, RSP=8, PLAN=1)),
     # TAIL: where the last round of tiles (128 output columns each) is at most a quarter full
-    # ((2048, 17408): 1088 tiles), the whole rounds, then the rest on ILV_TAIL tiles
+    # ((2048, 17408): 1088 tiles), the whole rounds, then the rest on 128 x 128 tiles
     (1 << 30, 0, "gi256x256k64w4r8t", "ilv",
      dict(BM=256, BN=256, BK=64, WM=2, WN=2, STAGES=2, GROUP=8, XCD=1, RSP=8, TAIL=1, PLAN=1)),
 ]
-
-# the tail tiles of the gate/up TAIL row: BM, BN, BK, WM, WN, STAGES of k_gemm_ilv (no split)
-ILV_TAIL = {1: (128, 128, 64, 2, 2, 3)}
 
 
 def _table(M):
@@ -197,7 +196,20 @@ def plan_tiles(M, cols, K, f=0, split=True):
 def plan(M, N, K, gate_up=False, split=True):
     """What a PLAN row's plan holds: (us, index into PLAN_TILES, splits), or None where no tile
     fits."""
-    return plan_tiles(M, 2 * N if gate_up else N, K, 0, split)  # tiles cover the rows of B
+    cols = 2 * N if gate_up else N  # tiles cover the rows of B
+    best = plan_tiles(M, cols, K, 0, split)
+    if best and gate_up and M <= 128 and best[2] > 1:  # ilv_plan of launch_prefill.h from here on
+        flat = plan_tiles(M, cols, K, 0, False)
+        if flat and best[0] > 0.9 * flat[0]:
+            best = flat
+    if best and gate_up and best[1:] == (5, 1) and N % 256 and K % 4096 == 0:
+        best = best[0], 2, 1
+    nm5, nm = -(-M // 192), -(-M // 256)
+    if best and best[1:] == (5, 1) and K >= 3584 and nm5 >= 8 and nm5 % 8:
+        us = tile_us(M, cols, K, 256, 256, 64, dict(_table(M)[5])[2][0])
+        if 2e-9 * M * cols * K > us or (nm % 8 == 0 and 0 < nm * (cols // 256) % 256 <= 32):
+            return us, 2, 1
+    return best
 
 
 # Divisibility each kind needs (checked at run time by dispatch.inc, mirrored here).

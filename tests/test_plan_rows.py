@@ -70,10 +70,13 @@ def _line_us(M, N, K, p):
     sn = p.get("SN", 1)
     wgs = N // (16 * sn)
     ks = _kslices(wgs, K, p["KS"]) if p.get("KS", 1) > 1 else 1
-    rows = 16 * sn + ((16 + M) // 2 if p["MB"] == 1 else M)
     w = wgs * ks
-    return 3 + (0.103 if p["MB"] == 1 else 0.095) * wgs * K * 2e-6 * rows * (
-        -(-w // 256) * 256) / w + (5 if ks > 1 else 0)
+    rounds = -(-w // 256)
+    if p["MB"] == 1 and rounds == 1:
+        return 2.5 + 1.5 * w / 256 + (0.89 + 0.037 * M) * K * 1e-3
+    if p["MB"] == 1:
+        return 5.8 + rounds * (1.1 + 0.029 * M) * K * 1e-3
+    return 3 + 0.095 * wgs * K * 2e-6 * (16 * sn + M) * rounds * 256 / w + (5 if ks > 1 else 0)
 
 
 def _choice(op, row, M, N, K):
@@ -88,24 +91,31 @@ def _choice(op, row, M, N, K):
         return "tail" if tail else (tile, sp)
     plan = sel.plan_tiles(M, N, K, f)
     if kind == "ilv" and not row.get("SW"):
-        return plan[1:]
+        return F16.plan(M, N, K)[1:]
     if plan is None:
         return "own"
+    us, tile, sp = plan
     if kind == "line" and op == 0:
         own, ahead = _line_us(M, N, K, row), 0.88
         if M <= 32 and K % 8192 == 0:
             return "own"
+        if row["MB"] == 1:
+            bm, bn = sel.PLAN_TILES[tile][:2]
+            us = max(us + 0.01 * -(-M // bm) * (N // bn) * sp, 0.46e-6 * N * K)
+            ahead = 0.93
     else:
         if kind == "line":
             bm, bn, bk = 16 * row["MB"], 16 * row["R"] * row.get("SN", 1), 128
         else:
             bm, bn, bk = row["BM"], row["BN"], row["BK"]
-        sp = _own(row, M, N, K) or 1
+        own_sp = _own(row, M, N, K) or 1
         rates = row["RATE"] if isinstance(row["RATE"], tuple) else (row["RATE"],)
-        rates = row.get("RATES", rates) if sp > 1 else rates
-        own = sel.tile_us(M, N, K, bm, bn, bk, rates[f], sp)
-        ahead = 0.85 if kind == "dma" and M <= 128 else 0.95
-    return plan[1:] if plan[0] < ahead * own else "own"
+        rates = row.get("RATES", rates) if own_sp > 1 else rates
+        own = sel.tile_us(M, N, K, bm, bn, bk, rates[f], own_sp)
+        ahead = 0.95
+        if kind == "dma":
+            ahead = (0.7 if K % 8192 == 0 else 0.85) if M <= 128 else 0.8 if sp > 1 else 0.95
+    return (tile, sp) if us < ahead * own else "own"
 
 
 def _check(op, shapes):
@@ -161,13 +171,24 @@ def test_w8a16_plans_agree(fmt):
 
 def test_fp16_plans_agree():
     few = [(M, N, K) for _, N, K in SWEEP if _ == 33 for M in (2, 8, 16, 17, 24, 32, 48)]
-    met = _check(0, SWEEP + few + [(16, 4096, 8192), (32, 5120, 16384)])  # rows 16 KiB apart
+    # (rows 16 KiB apart; 256-row tiles with a nearly empty last round)
+    met = _check(0, SWEEP + few + [(16, 4096, 8192), (32, 5120, 16384), (2048, 9216, 3840),
+                                   (2048, 17408, 5120), (2048, 9216, 2560), (2048, 10240, 3840),
+                                   (2048, 11264, 13824), (3000, 11008, 11008), (65, 15360, 8192)])
+    assert F16.plan(2048, 9216, 3840)[1] == 2 and F16.plan(2048, 10240, 3840)[1] == 5
+    assert F16.plan(2048, 11264, 13824)[1] == 2 and F16.plan(3000, 11008, 11008)[1] == 5
     assert {"split", "unsplit", "own line", "own dma", "own ilv"} <= set(met), met
-    for M, N, K in SWEEP:
-        row = F16.select_gate_up("gemm_gate_up", M, N, K)
-        if row and row.get("PLAN") and not (M > 128 and W8.tail_split(M, N, 256, 128)):
-            _, _, sp = F16.plan(M, N, K, gate_up=True)
-            assert _gate_up_need(0, M, N, K) == (0 if sp == 1 else sp * M * 2 * N * 4), (M, N, K)
+    shapes = [x for x in SWEEP + [(74, 17408, 3840), (700, 14464, 4096), (384, 13440, 8192)]
+              if (F16.select_gate_up("gemm_gate_up", *x) or {}).get("PLAN")
+              and not (x[0] > 128 and W8.tail_split(x[0], x[1], 256, 128))]
+    for (M, N, K), got in zip(shapes, record([dict(op=3, M=M, N=N, K=K, entry="ws")
+                                              for M, N, K in shapes])):
+        _, tile, sp = F16.plan(M, N, K, gate_up=True)
+        first = got["launches"][0]
+        assert tuple(first["args"][:6]) == F16.PLAN_TILES[tile][:6], (M, N, K)
+        assert len(got["launches"]) == 1 + (sp > 1), (M, N, K)
+        assert _gate_up_need(0, M, N, K) == (0 if sp == 1 else sp * M * 2 * N * 4), (M, N, K)
+    assert F16.plan(74, 17408, 3840, True)[2] == 1 and F16.plan(700, 14464, 4096, True)[1] == 2
 
 
 CASES = [  # M, N, K
