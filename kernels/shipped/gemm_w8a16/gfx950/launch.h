@@ -652,11 +652,15 @@ inline hipError_t launch_line_or_phase(const W8A16Params& p, hipStream_t s, cons
     return launch_line<MB, R, D, SN, WAVES>(p, s);
   }
 }
-// A tail-grid row of int8 weights, or the phase kernel of NS slabs where that fits: M = 32, us,
-// (34816, 5120) 37.8 against 34.5, gate/up (17408, 5120) 39.0 against 35.
+// A tail-grid row of int8 weights, or the phase kernel of NS slabs where that fits: NS = 9 serves 132
+// to 144 rows a CU, N = 33792 .. 36864 (gate/up: 17408 and 18432 output columns), the widths measured;
+// other widths stay on the line rows.  The phase kernel's launch costs more, so short K stays too.
+// us, M = 32, line -> phase: (34816, 5120) 37.7 -> 33.8, gate/up (17408, 5120) 38.9 -> 34.1; M = 17 ..
+// 32, line / phase times, means: K = 1024 0.90, 2048 0.94, 3072 1.00, 4096 1.15 to 12288; gate/up
+// 0.94, 0.97, 1.04, 1.23.
 template <int MB, int R, int D, int SN, int WAVES, int EPI, int NS>
 inline hipError_t launch_tail_or_phase(const W8A16Params& p, hipStream_t s) {
-  if (p.K < 12288 && (EPI ? phase_gu_fits<MB, NS, 4>(p) : phase_fits<MB, NS, 4>(p)))
+  if (p.K >= (EPI ? 3072 : 4096) && p.K < 12288 && (EPI ? phase_gu_fits<MB, NS, 4>(p) : phase_fits<MB, NS, 4>(p)))
     return launch_phase<MB, NS, 4, EPI>(p, s);
   return launch_line<MB, R, D, SN, WAVES, EPI, 1>(p, s);
 }

@@ -88,7 +88,7 @@ LADDER = [
     (16, 0, "l1r1n2d2", "line", dict(MB=1, R=1, D=2, SN=2, W=2048, PHASE=3.5)),
     # M <= 32, uint8: 1.11x the tail grid below at (32, 34816, 5120); int8 takes it from there
     (32, 12288, "p2n9d4", "phase", dict(MB=2, NS=9, D=4, KMAX=12288, fmts=(2,))),
-    # (int8: PHASE slabs, the same kernel as the row above where it fits)
+    # (int8: PHASE slabs, the same kernel as the row above where it fits and K >= 4096)
     (32, 12288, "l2r1n8d2t", "line", dict(MB=2, R=1, D=2, SN=8, W=2048, TL=1, PHASE=9)),
     (32, 12288, "l2r1n4d4", "line", dict(MB=2, R=1, D=4, SN=4, W=2048)),
     # long K: k slices, eight slab waves per activation ring (1.37x / 1.46x the row below at
@@ -221,7 +221,8 @@ LADDER_GATE_UP = [
     (16, 12288, "gl1r1n4d2t", "line", dict(MB=1, R=1, D=2, SN=4, W=2048, TL=1)),
     (16, 12288, "gl1r1n4d3", "line", dict(MB=1, R=1, D=3, SN=4, W=2048)),
     (16, 0, "gl1r1n2d4", "line", dict(MB=1, R=1, D=4, SN=2, W=2048)),
-    # M <= 32, uint8: 1.13x the tail grid below; int8 takes the same kernel from there (PHASE)
+    # M <= 32, uint8: 1.13x the tail grid below; int8 takes the same kernel from there (PHASE, K >=
+    # 3072)
     (32, 12288, "gp2n9d4", "phase", dict(MB=2, NS=9, D=4, KMAX=12288, fmts=(2,))),
     (32, 12288, "gl2r1n8d2t", "line", dict(MB=2, R=1, D=2, SN=8, W=2048, TL=1, PHASE=9)),
     (32, 12288, "gl2r1n4d2", "line", dict(MB=2, R=1, D=2, SN=4, W=2048)),

@@ -122,3 +122,19 @@ def test_sliced_against_oracle(gpu, fmt, case):
         r = O.rel_l2(host(C), ref)
         say("  relL2 %.3e" % r)
         assert r <= 5e-4
+
+
+def test_int8_tail_rows_take_the_phase_kernel_where_it_is_faster():
+    """M = 17 .. 32, int8: nine slabs and 4096 <= K < 12288 (gate/up: 3072)."""
+    cases = [  # op, N, K, phase
+        (1, 34816, 4096, True), (1, 34816, 3072, False), (1, 34816, 1024, False),
+        (1, 34816, 11264, True), (1, 34816, 12288, False), (1, 36864, 5120, True),
+        (1, 32768, 5120, False), (1, 34816, 4224, False),
+        (4, 17408, 3072, True), (4, 17408, 2048, False), (4, 18432, 5120, True),
+        (4, 17408, 12288, False), (4, 16384, 5120, False),
+    ]
+    got = record([dict(op=op, M=M, N=N, K=K) for op, N, K, _ in cases for M in (17, 32)])
+    for i, (op, N, K, phase) in enumerate(cases):
+        for g in got[2 * i:2 * i + 2]:
+            assert [l["kernel"] for l in g["launches"]] == [
+                "k_stream_phase" if phase else "k_stream_line"], (op, N, K)
