@@ -118,8 +118,10 @@ LADDER = [
     # ahead and gets its workspace.  64-row tiles: (64, 34816, 5120) 79 -> 54 / 76 -> 62 us (int8 /
     # uint8; at N = 15360 one round of the line row stays ahead), (33, 5120, 17408) 34 -> 28 / 37 ->
     # 34, (64, 2560, 2560) 16.5 -> 11
+    # (RATE, one round at long K: int8 4.4 .. 4.9, uint8 4.3 .. 4.6.  int8 plans are faster than
+    # estimated, 5.5 keeps what they gain; uint8 ones slower: (33, 14208, 12928) 57 us here, 72 planned)
     (64, 12288, "l4r1n4d3", "line",
-     dict(MB=4, R=1, D=3, SN=4, W=2048, PLAN=1, RATE=(5.5, 5.5))),
+     dict(MB=4, R=1, D=3, SN=4, W=2048, PLAN=1, RATE=(5.5, 4.8))),
     # 32 < M <= 64, narrow N and long K: the int8 interleaved kernel on 128 x 256 tiles of 128 k
     # (whole weight lines) with split-K (1.09x the 64-k tile row at (64, 5120, 17408), which was
     # 1.3x the line row)

@@ -191,6 +191,18 @@ def test_fp16_plans_agree():
     assert F16.plan(74, 17408, 3840, True)[2] == 1 and F16.plan(700, 14464, 4096, True)[1] == 2
 
 
+def test_line_row_keeps_its_uint8_rounds():
+    """At 32 < M <= 64 one round of the line row streams uint8 weights at 4.4 .. 4.6 us per 1000 k at
+    long K; a plan that is not faster than that stays out ((33, 14208, 12928) 57 us against 72)."""
+    line = [(33, 14208, 12928), (64, 13696, 13312), (48, 14208, 17408), (50, 13824, 6144)]
+    planned = [(64, 34816, 5120), (48, 20480, 17408), (33, 27648, 13824)]
+    for (M, N, K), got in zip(line + planned, record([dict(op=2, M=M, N=N, K=K, entry="pool")
+                                                      for M, N, K in line + planned])):
+        tag = capi.route(2, M, N, K)
+        assert tag == "l4r1n4d3"
+        assert (got["launches"][0]["kernel"] == "k_stream_line") == ((M, N, K) in line), (M, N, K)
+
+
 CASES = [  # M, N, K
     (9, 5120, 2560),     # 64-row tiles, most rows past M (fp16)
     (33, 5120, 1152),
