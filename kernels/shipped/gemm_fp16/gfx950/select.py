@@ -27,8 +27,8 @@ ARCH = "gfx950"
 
 # Tiles a PLAN row chooses from (interleaved kernel): BM, BN, BK, WM, WN, STAGES, split-K
 # instantiated.  PLAN_TABLES: M_max, us a round, a split, a MB of partial sums adds, us a million
-# weights take at least, and (tile, us
-# per 1000 k of one round).  plan() below and plan_tiles of the frozen kernel file state the rule.
+# weights take at least, and (tile, us per 1000 k of one round).  plan() below and plan_tiles of
+# the frozen kernel file state the rule.
 PLAN_TILES = (
     (128, 128, 64, 2, 2, 4, 1),
     (128, 256, 64, 1, 4, 3, 1),

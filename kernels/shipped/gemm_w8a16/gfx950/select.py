@@ -14,9 +14,8 @@ FORMATS = (1, 2)
 
 # Tiles a PLAN row chooses from (interleaved kernel): BM, BN, BK, WM, WN, STAGES, split-K
 # instantiated.  PLAN_TABLES: M_max, us a round, a split, a MB of partial sums adds, us a million
-# weights take at least, and (tile, us
-# per 1000 k of one round (int8, uint8)).  plan() below and plan_tiles of the frozen kernel file
-# state the rule.
+# weights take at least, and (tile, us per 1000 k of one round (int8, uint8)).  plan() below and
+# plan_tiles of the frozen kernel file state the rule.
 PLAN_TILES = (
     (128, 128, 128, 1, 4, 2, 1),
     (128, 256, 128, 1, 4, 2, 1),
@@ -115,9 +114,9 @@ LADDER = [
     (32, 0, "h32r1u4n2", "shared", dict(MB=2, R=1, U=4, SN=2, TPB=512)),
     # 32 < M <= 128: PLAN with the row's own rate (RATE, us per 1000 k and round of int8 / uint8) or,
     # for a split-K row, its own tile and split count: the plan runs where it is estimated 5 %
-    # ahead and gets its workspace.  64-row tiles: (64, 34816, 5120) 79 -> 54 / 76 -> 62 us (int8 /
-    # uint8; at N = 15360 one round of the line row stays ahead), (33, 5120, 17408) 34 -> 28 / 37 ->
-    # 34, (64, 2560, 2560) 16.5 -> 11
+    # ahead and gets its workspace.  64-row tiles: (64, 34816, 5120) 77 -> 54 / 77 -> 62.6 us (int8 /
+    # uint8; at N = 15360 one round of the line row stays ahead), (33, 5120, 17408) 33 -> 28 / 39 ->
+    # 35, (64, 2560, 2560) 17 -> 12
     # (RATE, one round at long K: int8 4.4 .. 4.9, uint8 4.3 .. 4.6.  int8 plans are faster than
     # estimated, 5.5 keeps what they gain; uint8 ones slower: (33, 14208, 12928) 57 us here, 72 planned)
     (64, 12288, "l4r1n4d3", "line",
@@ -161,17 +160,17 @@ LADDER = [
           fmts=(2,))),
     # 64 < M <= 128: 128 x 256 tiles (one tile row), split-K where the column tiles are too few
     # to fill the part (the variant driver's rows: 1.5-2.9x the line and register-staged rows)
-    # (RATE of a split grid: 60 tiles in four splits take 35 us at (128, 15360, 3840), 120 unsplit
-    # tiles of 64 rows 30; unsplit, at N = 34816, the row is its own best)
+    # (RATE of a split grid: 60 tiles in four splits take 34.5 us at (128, 15360, 3840), 120 unsplit
+    # tiles 28; unsplit, at N = 34816, the row is its own best)
     (128, 0, "i8x128x256s3w256", "ilv8",
      dict(BM=128, BN=256, BK=64, WM=1, WN=4, STAGES=3, GROUP=8, XCD=1, RSP=8, SW=256, MINKT=8,
           PLAN=1, RATE=(13.1, 14.0), RATES=(22.0, 24.0))),
     (128, 0, "l8r1n2d3", "line", dict(MB=8, R=1, D=3, SN=2, W=2048, NMAX=12288)),
     # PLAN rows: where K % 128 == 0 the launcher picks the tile and the split count by plan(); the
     # row's own tile names it and runs what the plan does not fit.  At (256, 5120, 17408) 128 x 256
-    # tiles in six splits take 62 / 66 us, the register-staged 128 x 128 tiles 235 / 281 (int8 /
-    # uint8); over M = 160 .. 4096 and N = 1024 .. 34816 the plan is 1.55 / 1.59 times as fast as the
-    # single tiles (geometric mean)
+    # tiles in six splits take 62 / 66 us, the register-staged 128 x 128 tiles 246 / 288 (int8 /
+    # uint8).  Random shapes with the weights from HBM, single tiles against the plan, geometric means
+    # (int8 / uint8): 2.36 / 2.64x at 128 < M <= 256, 1.63 / 1.58x up to M = 1024, 1.09x from there
     (256, 0, "m128x128k64", "mfma",
      dict(BM=128, BN=128, BK=64, WM=2, WN=2, MS=32, SWZ=1, GROUP=8, XCD=1, PLAN=1)),
     # narrow N (fewer than 8 tiles of 256 columns): 256x256 tiles leave most CUs idle; 128 x 128
@@ -184,6 +183,8 @@ LADDER = [
     # 128-k)
     (1 << 30, 0, "m128x128k64s16", "mfma",
      dict(BM=128, BN=128, BK=64, WM=2, WN=2, MS=16, SWZ=1, GROUP=8, XCD=1, NMAX=2048, fmts=(1,))),
+    # (This row and the next run by plan() alike; the rule below decides which of the two names a
+    # shape, and the figures are those of the single tiles before the plan.)
     # FILL: where one round of 192 x 256 tiles holds the whole grid and has more tiles than the
     # 256 x 256 grid (220 against 160 tiles at (2048, 5120)), the 192-row tiles fill more of the
     # part: 1.05-1.10x the row below at (2048, 5120, 5120 | 6144 | 17408) in both formats,

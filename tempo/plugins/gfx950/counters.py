@@ -31,6 +31,7 @@ import contextlib
 import csv
 import glob
 import os
+import re
 import shutil
 import subprocess
 import tempfile
@@ -175,6 +176,16 @@ def assign_segments(dispatches: list, segments: list, match: str) -> dict:
                 got.append(d)
         out[seg["label"]] = got
     return out
+
+
+def kernel_name(symbol: str) -> str:
+    """A dispatch's kernel without its namespace, return type and arguments; rocprofv3 leaves the
+    names with _Float16 arguments mangled."""
+    m = re.search(r"\d(k_[a-z0-9_]+?)(?:I((?:L[a-z]+\d+E)+)E)?E", symbol)
+    if symbol.startswith("_Z") and m:
+        args = re.findall(r"L[a-z]+(\d+)E", m.group(2) or "")
+        return m.group(1) + ("<%s>" % ", ".join(args) if args else "")
+    return symbol.split("(")[0].split("::")[-1]
 
 
 def _median(xs):

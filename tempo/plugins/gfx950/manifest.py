@@ -301,7 +301,7 @@ def fold_counters(rows, counter_files, op, md5=None):
             c = by.get((row["M"], row["N"], row["K"], row["fmt"]))
             if c is not None:
                 row["counters"] = dict(c["counters"], groups=got.get("groups"),
-                                       route=c.get("route"))
+                                       route=c.get("route"), kernels=c.get("kernels"))
                 n += 1
     return n
 

@@ -135,6 +135,26 @@ CALIB_BYTES = 1 << 30
 REPS = 3
 
 
+def dispatches_per_launch(op, M, N, K, fmt) -> int:
+    """Kernels one call dispatches with a workspace at hand: a split-K call its main kernel, then
+    the reduction; a call whose N is in two parts, its two parts."""
+    from cuda_tempiler_amd import capi
+    from tempo.plugins.gfx950 import manifest
+
+    if op == "fmha":
+        return 1
+    need = capi.workspace_bytes(fmt, M, N, K)
+    if op == "gemm_w8a16":
+        sel = manifest._select(op)
+        row = sel.select(op, M, N, K, fmt=fmt)
+        if row.get("PLAN") and M > 128 and K % 128 == 0 and sel.plan(M, N, K, fmt)[3]:
+            return 2
+        route = capi.route(fmt, M, N, K)
+        if route.endswith("t2") and route.startswith("i8"):
+            return 3 if need else 2  # whole rounds, tail (+ reduce)
+    return 2 if need else 1
+
+
 def counter_pass(op: str, segfile: str, quick: bool = False) -> int:
     """The program a counter pass profiles: a calibration copy (3 x 1 GiB device copies), then
     REPS launches of the shipped kernel per configuration shape (inputs generated on the device
@@ -186,18 +206,8 @@ def counter_pass(op: str, segfile: str, quick: bool = False) -> int:
         for _ in range(REPS - 1):
             run()
         torch.cuda.synchronize()
-        # a split-K launch dispatches two kernels: its main kernel, then the reduction; a launch
-        # whose N is in two parts, its two parts
         route = capi.route(fmt, M, N, K) if op != "fmha" else "k_fmha_fwd"
-        per = 1 if op == "fmha" or capi.workspace_bytes(fmt, M, N, K) == 0 else 2
-        if op == "gemm_w8a16":
-            from tempo.plugins.gfx950 import manifest
-            sel = manifest._select(op)
-            row = sel.select(op, M, N, K, fmt=fmt)
-            if row.get("PLAN") and M > 128 and K % 128 == 0 and sel.plan(M, N, K, fmt)[3]:
-                per = 2
-            elif route.endswith("t2") and route.startswith("i8"):
-                per = 3 if capi.workspace_bytes(fmt, M, N, K) else 2  # whole rounds, tail (+ reduce)
+        per = dispatches_per_launch(op, M, N, K, fmt)
         segs.append(dict(label=label_of(M, N, K, fmt), count=REPS * per, per_launch=per,
                          route=route))
     with open(segfile, "w") as f:
@@ -209,10 +219,10 @@ def counters(op: str, out: str, groups, quick: bool = False) -> str:
     """Parent of the counter passes (never touches the GPU): one rocprofv3 --pmc run per group,
     then per-launch figures per configuration shape into out/counters_<op>.json."""
     from tempo.plugins.gfx950.counters import (Gfx950Meters, GROUPS, assign_segments,
-                                               copy_scales, derive, medians)
+                                               copy_scales, derive, kernel_name, medians)
 
     meters = Gfx950Meters()
-    per_shape, scales, routes, per_launch = {}, {}, {}, {}
+    per_shape, scales, routes, per_launch, kernels = {}, {}, {}, {}, {}
     for g in groups:
         d = os.path.abspath(os.path.join(out, "pmc_%s_%s" % (op, g)))
         seg = os.path.join(d, "segments.json")
@@ -232,6 +242,8 @@ def counters(op: str, out: str, groups, quick: bool = False) -> str:
             if s["label"] in got:
                 routes[s["label"]] = s.get("route")
                 per_launch[s["label"]] = s.get("per_launch", 1)
+                kernels[s["label"]] = [kernel_name(d["kernel"]) for d in
+                                       got[s["label"]][:s.get("per_launch", 1)]]
                 per_shape.setdefault(s["label"], {}).update(
                     medians(got[s["label"]], s.get("per_launch", 1)))
     rows = []
@@ -242,6 +254,7 @@ def counters(op: str, out: str, groups, quick: bool = False) -> str:
             fig["pmc_duration_us"] = med["_duration_ns"] / 1e3
         rows.append(dict(M=M, N=N, K=K, fmt=fmt, route=routes.get(lab),
                          dispatches_per_launch=per_launch.get(lab, 1),
+                         kernels=kernels.get(lab),
                          algorithmic_bytes=algorithmic_bytes(op, M, N, K, fmt),
                          algorithmic_flops=algorithmic_flops(op, M, N, K, fmt),
                          counters=fig))
@@ -287,6 +300,12 @@ def render_counters(path: str) -> str:
             f(c.get("traffic_over_algorithmic"), "%.2f"), f(c.get("mfma_util_spec_clock"), "%.3f"),
             f(c.get("mfma_util") if long_ else None, "%.3f"),
             f(c.get("sclk_ghz") if long_ else None, "%.2f"), f(lds, "%.3f"), f(confl, "%.3f")))
+    if any(r.get("kernels") for r in got["rows"]):
+        lines += ["", "Kernels of one launch (the row names the shape; its plan or its other arm may "
+                  "run it):", ""]
+        lines += ["    %d,%d,%d,%d: %s" % (r["M"], r["N"], r["K"], r["fmt"],
+                                           " + ".join(r.get("kernels") or ["-"]))
+                  for r in got["rows"]]
     lines += ["", "Exact HBM bytes per launch (M,N,K,fmt: fetch, write, total, algorithmic):", ""]
     for r in got["rows"]:
         c = r["counters"]

@@ -141,8 +141,12 @@ inline int split_count(int tiles, int ktiles, int slots, int minkt) {
 // least estimated time.  A table serves the rows up to m_max: microseconds per 1000 k of one round
 // of a tile (one workgroup on each of the 256 CUs; per weight format), and what a round, a split
 // (its second kernel) and a MB of partial sums (written and read) add.  The figures are fits to
-// measured grids (100 .. 2200 workgroups; N = 1024 .. 34816, K = 2560 .. 17408): the pick is within
-// 1 % (M > 128) and 2-5 % (below) of the fastest tile and split count, geometric mean.
+// measured grids (100 .. 2200 workgroups; N = 1024 .. 34816, K = 2560 .. 17408) and order the
+// alternatives only.  As times they are low: over random shapes at M > 64 with the weights from HBM
+// splits take 1.16 times as long (median of 2054; 1.00 to 1.34 at the 5th and 95th percentile),
+// unsplit tiles 1.09 times (of 2675; 0.91 to 1.67, the latter at short K) -- (200, 15360, 3840) fp16
+// 42 us for 34, (2048, 2 x 17408, 5120) int8 620 for 501 -- for a round's rate depends on the clock
+// under load and, below M = 256, on the HBM.
 struct TileDims {
   int bm, bn, bk;
   bool splits;  // instantiated with split-K (the 256 x 256 tiles spill with it)

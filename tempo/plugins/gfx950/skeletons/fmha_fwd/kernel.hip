@@ -126,9 +126,10 @@ __device__ __forceinline__ void fmha_buf_lds16(const void* base, unsigned nrec, 
 // groups).  256-row tiles on eight waves and 64 rows per wave were within 3 % of the two-workgroup
 // form, and reading the next block's first fragments at the end of the chain within 1 %.
 //
-// `Hg` head groups of G = H / Hg query heads, gk = Hg / Hkv groups a KV head: Hg = Hkv packs the query
-// heads of a KV head as above; Hg = H gives every head tiles of its own, for grids that leave CUs idle and have few key blocks.  There a workgroup's time is its CU's
-// intake of Q and store of O (64 KiB each for 128 rows at D = 256), which packing only concentrates
+// `Hg` head groups of G = H / Hg query heads, gk = Hg / Hkv groups a KV head: Hg = Hkv packs the
+// query heads of a KV head as above; Hg = H gives every head tiles of its own, for grids that leave
+// CUs idle and have few key blocks.  There a workgroup's time is its CU's intake of Q and store of O
+// (64 KiB each for 128 rows at D = 256), which packing only concentrates
 // (us, packed -> one head a tile, D = 256: 4 sequences x 64 rows and keys, 16 heads, 8 KV heads
 // 12.3 -> 9.9; 1 x 16 rows x 203 keys, 64 heads 16.9 -> 13.1).
 //

@@ -19,7 +19,7 @@
 // through LDS in chunk order, written as fp16 into an LDS image of the workgroup's output columns,
 // and stored row by row.  The sums take the rings' and the staging's LDS (red_units of 1 KiB per
 // wave, all of them in one or two rounds): one slab per round with a barrier in each cost 2 to 4
-// us a launch (M = 32, 34816 x 5120 uint8: 38.8 us, now 33.9; M = 16: 33.0, now 31.1).
+// us a launch (M = 32, 34816 x 5120 uint8: 38.8 us, now 34.7; M = 16: 32.9, now 31.3).
 // Activations: MB = 1 / 2 (M <= 16 / 32): a phase ahead, four copies per 16 rows (rows past M
 // re-read row M-1), each of 4 rows x 256 bytes -- whole lines, as the weights: a copy in the
 // fragment layout takes half of 16 lines, and the 4 MB of them cost as many line requests a phase

@@ -84,3 +84,20 @@ def test_strided_w8_cases_route_as_named():
         for tag, M, N, K, pa, pb, pc in cases:
             assert route(M, N, K)["tag"] == tag, (name, M, N, K)
             assert pa % 8 == 0 and pb % (8 if name.startswith("fp16") else 16) == 0 and pc % 4 == 0
+
+
+def test_counter_step_counts_every_dispatch():
+    """A counter pass attributes dispatches to shapes in launch order: the count it expects of a
+    call is the count of kernels the compiled dispatch launches."""
+    from tempo.plugins.gfx950 import measure_shipped as ms
+
+    for op in ("gemm_fp16", "gemm_w8a16"):
+        shapes = list(ms.cases_of(op))
+        for (M, N, K, fmt), got in zip(shapes, record([dict(op=fmt, M=M, N=N, K=K, entry="pool")
+                                                       for M, N, K, fmt in shapes])):
+            assert got["rc"] == 0 and len(got["launches"]) == ms.dispatches_per_launch(
+                op, M, N, K, fmt), (op, M, N, K, fmt)
+    for S, H, D, Hkv in ms.cases_of("fmha"):
+        got, = record([dict(fmha=[1, S, S, H, Hkv, D, 1], entry="pool")])
+        assert got["rc"] == 0 and len(got["launches"]) == ms.dispatches_per_launch(
+            "fmha", S, H, D, Hkv), (S, H, D, Hkv)

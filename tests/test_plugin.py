@@ -386,3 +386,16 @@ def test_counter_step_attribution_and_figures(tmp_path):
 
     with _pt.raises(RuntimeError):
         C.assign_segments(disp, segs + [dict(label="c", count=1)], "tempo")
+
+
+def test_kernel_names_of_dispatches():
+    from tempo.plugins.gfx950.counters import kernel_name
+
+    for symbol, want in (
+            ("void tempo::gen8::k_stream_line<2, 1, 2, 1, 0, 1, 256, 0>(_Float16 const*)",
+             "k_stream_line<2, 1, 2, 1, 0, 1, 256, 0>"),
+            ("_ZN5tempo4gen815k_splitk_reduceILi4EEEvPKfiiiPDF16_i", "k_splitk_reduce<4>"),
+            ("_ZN10tempo_fmha4fmha10k_fmha_fwdILi256ELb1ELi1EEEvPKDF16_S3_",
+             "k_fmha_fwd<256, 1, 1>"),
+            ("tempo::gen::k_fill(float*)", "k_fill")):
+        assert kernel_name(symbol) == want
