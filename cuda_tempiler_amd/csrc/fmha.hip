@@ -68,8 +68,12 @@ static size_t ws_bytes(const TempoFmhaParams& p, const Plan& pl) {
 //     3.5 (5 at D = 256) for the second kernel (512 rows over 8192 keys, 16 heads, D = 256: 96
 //     against 265; 2 x 158 rows over 235 keys, 2 heads, D = 256: 18.5 cut, 16.9 whole).
 //   * Tiles of one head each where a round of the CUs holds them, they have few key blocks and no
-//     cut pays: a tile's Q and O pass its CU at 40 GB/s (qo), so 128 packed rows cost 3.3 at D = 256
-//     and 38 rows 1.0 (4 x 38 rows x 104 keys, 8 heads, 2 KV heads: 14.3 packed, 10.6 apart).
+//     cut pays.  Either form is its longest tile -- 0.65 (D = 128) or 1.3 a block, and its rows' Q and
+//     O, which pass the tile's CU at 40 GB/s -- and the key blocks all its tiles bring in, 0.034 or
+//     0.068 a MB: 4 x 38 rows x 104 keys, 8 heads, 2 KV heads, D = 256: 14.3 packed, 10.6 apart;
+//     32 x 107 x 107, 8 heads, 1 KV head: 14.9 packed, 18.5 apart.  Of 6694 random calls of both
+//     forms 73 take over 3 % more than packed and 24 than apart (693 and none by the longest tile
+//     alone, counted as whole).
 static Plan plan(const TempoFmhaParams& p) {
   constexpr int kCus = 256;
   const int G = p.H / p.Hkv;
@@ -80,13 +84,24 @@ static Plan plan(const TempoFmhaParams& p) {
   const long tiles = bh * (pl.rows ? 1 : (R + fmha::BQ - 1) / fmha::BQ);
   if (!pl.rows && p.D == 128 && tiles <= 2 * kCus && L >= 16) pl.kg = 2;
   const double blk = p.D == 128 ? 0.47 : 1.07;
-  // a tile of r rows' Q and O; the longest tile of one head, in the last rows or the 128 before them
-  auto qo = [&](long r) { return (double)(r < fmha::BQ ? r : fmha::BQ) * p.D * 1e-4; };
-  const int nq = (p.Sq + fmha::BQ - 1) / fmha::BQ, last = p.Sq - (nq - 1) * fmha::BQ;
-  double own = L * blk + qo(last);
-  if (nq > 1) own = std::max(own, (L - (p.causal ? (last + 31) / 32 : 0)) * blk + qo(fmha::BQ));
-  pl.apart = !pl.rows && pl.kg == 1 && G > 1 && L <= 16 && (long)p.B * p.H * nq <= kCus &&
-             own < L * blk + qo(R);
+  const int nq = (p.Sq + fmha::BQ - 1) / fmha::BQ;
+  double gain = 0;  // of tiles of one head over packed ones, where they are the better
+  if (!pl.rows && pl.kg == 1 && G > 1 && L <= 16 && (long)p.B * p.H * nq <= kCus) {
+    auto form = [&](int rows, int g, long groups) {  // `groups` times the tiles of `rows` rows
+      double longest = 0;
+      long blocks = 0;
+      for (int r0 = 0; r0 < rows; r0 += fmha::BQ) {
+        const int n = rows - r0 < fmha::BQ ? rows - r0 : fmha::BQ;
+        const int l = p.causal ? fmha::fmha_tile_blocks<true>(r0, n, rows, g, p.Sq, p.Sk)
+                               : fmha::fmha_tile_blocks<false>(r0, n, rows, g, p.Sq, p.Sk);
+        longest = std::max(longest, l * (p.D == 128 ? 0.65 : 1.3) + n * p.D * 1.56e-4);
+        blocks += l;
+      }
+      return longest + (p.D == 128 ? 0.034 : 0.068) * groups * blocks * 128 * p.D * 1e-6;
+    };
+    gain = form((int)R, G, bh) - form(p.Sq, 1, (long)p.B * p.H);
+    pl.apart = gain > 0;
+  }
   if (2 * tiles > kCus) {
     if (pl.apart) pl.hg = p.H;
     return pl;
@@ -101,7 +116,7 @@ static Plan plan(const TempoFmhaParams& p) {
   int best = 1;
   for (int n = 2; n <= 64 && n * tiles <= kCus && 4 * n <= L; ++n)
     if (cost(n) < cost(best)) best = n;
-  if (pl.apart && own <= cost(best) + qo(R)) {
+  if (pl.apart && (best == 1 || gain - 1 >= cost(1) - cost(best))) {  // (1: the estimates' error)
     pl.hg = p.H;
     return pl;
   }

@@ -47,6 +47,9 @@ def test_strided_gpu_cases_reach_every_form():
     ((1, 8, 96, 4, 1, 256, True), 4),              # few rows, few blocks: not the few-rows kernel
     ((1, 8, 160, 4, 1, 256, True), 1),             # its five blocks: that kernel
     ((4, 38, 104, 8, 8, 256, True), 4 * 8),        # nothing to pack
+    ((32, 107, 107, 8, 1, 256, True), 32 * 7),     # a full part: packed tiles bring in fewer keys
+    ((2, 101, 101, 16, 2, 128, True), 2 * 2 * 7),  # packed causal tiles are shorter
+    ((2, 40, 101, 16, 2, 128, True), 2 * 16),
 ])
 def test_which_tiles_pack_heads(case, tiles):
     """Without a workspace: one workgroup per (batch, head group, tile)."""
