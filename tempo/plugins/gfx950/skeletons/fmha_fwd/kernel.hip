@@ -69,7 +69,7 @@ __device__ __host__ __forceinline__ int fmha_tile_blocks(int r0, int rows, int R
   int kend = Sk;
   if (CAUSAL) {
     const int end = r0 + rows < R ? r0 + rows : R;
-    const int seen = (G == 1 ? end - 1 : (end - 1) / G) + 1 + Sk - Sq;  // by the tile's last row
+    const int seen = (end - 1) / G + 1 + Sk - Sq;  // keys the tile's last row sees
     kend = seen < Sk ? seen : Sk;
     if (kend < 0) kend = 0;
   }
@@ -226,7 +226,8 @@ __global__ __launch_bounds__(256 * KG, D == 128 && KG == 1 ? 2 : 1) void k_fmha_
   // the tile's key blocks, this workgroup's [lo, lo + nwg), and this key group's: the groups take
   // ceil(nwg / KG) blocks each; where the last has fewer, its blocks past the range re-read the
   // last one and are masked, so that every group meets the same barriers
-  const int nkt = fmha_tile_blocks<CAUSAL>(r0, BQW, R, G, Sq, Sk);
+  const int nkt = G == 1 ? fmha_tile_blocks<CAUSAL>(r0, BQW, R, 1, Sq, Sk)
+                         : fmha_tile_blocks<CAUSAL>(r0, BQW, R, G, Sq, Sk);
   const int wlo = sp * chunk;
   if (sp > 0 && wlo >= nkt) return;
   const int nwg = min(nkt - wlo, chunk);
