@@ -118,8 +118,9 @@ hipError_t run_plan(const GemmParams& p, hipStream_t s, float* ws, const TilePla
 // groups of 8 and a ragged one: those run at 0.82 to 1.05 PFLOP/s, whatever their round's fill, where
 // 256 x 256 tiles (2) in whole groups reach 1.1.  So from K = 3584 on the 256-row tiles take what the
 // 192-row ones would need longer for at 1 PFLOP/s, and what leaves their own last round of whole
-// groups at most 32 tiles (us, 256 rows against 192: (2048, 11008, 11008) 478, 539; (2048, 11264,
-// 13824) 582, 660; (2048, 9216, 12288) 491, 516; (2048, 17408, 11008) 724, 871; where they stay:
+// groups at most 48 tiles (us, 256 rows against 192: (2048, 11008, 11008) 478, 539; (2048, 11264,
+// 13824) 582, 660; (2048, 9216, 12288) 491, 516; (2048, 17408, 11008) 724, 871; (2048, 9472, 14080)
+// 570, 644; (2048, 9728, 4352) 177, 187; where they stay:
 // (2048, 10240, 3584) 162, 141; in whole groups: (3000, 11008, 11008) 819, 628).
 // Fused gate/up (cols = 2N): at M <= 128 a split has to be 10 % ahead of the best unsplit tile, whose
 // short last round costs less than a whole one ((74, 17408, 3840) 66 us unsplit, 71 in three splits);
@@ -139,7 +140,7 @@ inline TilePlan ilv_plan(const GemmParams& p, int cols, bool split) {
     if (r.tile == 2) rate = r.us[0];
   const double us = tile_us(plan_table(kPlanTables, p.M), rate, 256, 256, 64, p.M, cols, p.K, 1);
   const int rest = (int)((long)nm * (cols / 256) % 256);
-  if (2e-9 * p.M * cols * p.K > us || (nm % 8 == 0 && rest > 0 && rest <= 32)) {
+  if (2e-9 * p.M * cols * p.K > us || (nm % 8 == 0 && rest > 0 && rest <= 48)) {
     pl.tile = 2;
     pl.us = us;
   }

@@ -207,7 +207,7 @@ def plan(M, N, K, gate_up=False, split=True):
     nm5, nm = -(-M // 192), -(-M // 256)
     if best and best[1:] == (5, 1) and K >= 3584 and nm5 >= 8 and nm5 % 8:
         us = tile_us(M, cols, K, 256, 256, 64, dict(_table(M)[5])[2][0])
-        if 2e-9 * M * cols * K > us or (nm % 8 == 0 and 0 < nm * (cols // 256) % 256 <= 32):
+        if 2e-9 * M * cols * K > us or (nm % 8 == 0 and 0 < nm * (cols // 256) % 256 <= 48):
             return us, 2, 1
     return best
 

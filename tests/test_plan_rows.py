@@ -203,6 +203,14 @@ def test_line_row_keeps_its_uint8_rounds():
         assert (got["launches"][0]["kernel"] == "k_stream_line") == ((M, N, K) in line), (M, N, K)
 
 
+def test_nearly_empty_last_round_of_256_rows():
+    """Up to 48 tiles past the whole rounds 256-row tiles are the faster; past that 192-row ones."""
+    shapes = [(2048, 9472, 14080), (2048, 9728, 4352), (2048, 10240, 3584)]
+    for (M, N, K), rows, got in zip(shapes, (256, 256, 192), record([
+            dict(op=0, M=M, N=N, K=K, entry="pool") for M, N, K in shapes])):
+        assert got["launches"][0]["args"][:2] == [rows, 256], (M, N, K)
+
+
 CASES = [  # M, N, K
     (9, 5120, 2560),     # 64-row tiles, most rows past M (fp16)
     (33, 5120, 1152),
