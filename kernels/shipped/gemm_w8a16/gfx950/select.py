@@ -120,7 +120,7 @@ LADDER = [
     # (RATE, one round at long K: int8 4.4 .. 4.9, uint8 4.3 .. 4.6.  int8 plans are faster than
     # estimated, 5.5 keeps what they gain; uint8 ones slower: (33, 14208, 12928) 57 us here, 72 planned)
     (64, 12288, "l4r1n4d3", "line",
-     dict(MB=4, R=1, D=3, SN=4, W=2048, PLAN=1, RATE=(5.5, 4.8))),
+     dict(MB=4, R=1, D=3, SN=4, W=2048, PLAN=1, RATE=(5.5, 4.6))),
     # 32 < M <= 64, narrow N and long K: the int8 interleaved kernel on 128 x 256 tiles of 128 k
     # (whole weight lines) with split-K (1.09x the 64-k tile row at (64, 5120, 17408), which was
     # 1.3x the line row)
